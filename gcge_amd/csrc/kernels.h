@@ -77,6 +77,12 @@ void copy_cols(int64_t nrows, int ncols, const double *X, int64_t ldx, double *Y
                int64_t ldy, hipStream_t s);
 // out[c] = X[:, c] . Y[:, c]; partial is scratch of dots_scratch(ncols) doubles.
 int64_t dots_scratch(int ncols);
+// G[i + j ldg] = sum over c < nchunk of partial[c stride + off], in order of
+// c, for the entries of tm x tn tiles of TM x TN (off = (tile TM + i % TM) TN
+// + j % TN, tile = (i / TM) tn + j / TN, i < m, j < n); transposed stores
+// G[j + i ldg].
+void sum_chunks(int m, int n, int tm, int tn, int TM, int TN, int nchunk, const double *partial,
+                double *G, int ldg, bool transposed, hipStream_t s);
 void col_dots(int64_t nrows, int ncols, const double *X, int64_t ldx, const double *Y,
               int64_t ldy, double *out, double *partial, hipStream_t s);
 // G (m x n, ldg) = X^T Y with X: nrows x m, Y: nrows x n.  lower_only

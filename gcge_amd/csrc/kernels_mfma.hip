@@ -49,7 +49,7 @@ __device__ __forceinline__ d4 mfma(double a, double b, d4 c)
 // into registers before the current stage's MFMAs, so HBM latency overlaps
 // the matrix-core work; the default shape holds 98 VGPRs + 128 AGPRs, two
 // waves per SIMD.  Partial tiles per chunk are summed by
-// k_gram_mfma_reduce in a fixed order (deterministic, no atomics).  Each
+// sum_chunks in a fixed order (deterministic, no atomics).  Each
 // entry sums its rows in the same order whatever the shape; the chunking,
 // and so the rounding of the partial sums, follows the tile count.
 // ---------------------------------------------------------------------
@@ -180,25 +180,6 @@ __global__ __launch_bounds__(kWG) void k_gram_mfma(
                 const int jj = wn * 16 * NB + b * 16 + li;
                 out[ii * TN + jj] = acc[a][b][v];
             }
-}
-
-__global__ __launch_bounds__(kWG) void k_gram_mfma_reduce(int m, int n, int tm, int tn, int TM,
-                                                          int TN, int nchunk,
-                                                          const double *__restrict__ partial,
-                                                          double *__restrict__ G, int ldg)
-{
-    // threads walk the partial tiles in storage order, so each chunk's read
-    // is contiguous across the wavefront
-    const int64_t off = (int64_t)blockIdx.x * kWG + threadIdx.x;
-    const int64_t stride = (int64_t)tm * tn * TM * TN;
-    if (off >= stride) return;
-    const int t = (int)(off / (TM * TN));
-    const int within = (int)(off % (TM * TN));
-    const int i = (t / tn) * TM + within / TN, j = (t % tn) * TN + within % TN;
-    if (i >= m || j >= n) return;
-    double s = 0.0;
-    for (int c = 0; c < nchunk; ++c) s += partial[off + (int64_t)c * stride];
-    G[i + (int64_t)j * ldg] = s;
 }
 
 // Tile shape of a Gram of m x n (see k_gram_mfma).
@@ -446,9 +427,7 @@ void launch_gram(const GramPlanM &p, int64_t nrows, int m, int n, const double *
     else
         GCGE_GRAM(2, 4);
 #undef GCGE_GRAM
-    const int64_t total = (int64_t)p.tm * p.tn * p.tile_doubles();
-    k_gram_mfma_reduce<<<(unsigned)((total + kWG - 1) / kWG), kWG, 0, s>>>(
-        m, n, p.tm, p.tn, p.sh.rows(), p.sh.cols(), p.nchunk, partial, G, ldg);
+    sum_chunks(m, n, p.tm, p.tn, p.sh.rows(), p.sh.cols(), p.nchunk, partial, G, ldg, false, s);
 }
 
 }  // namespace

@@ -1,0 +1,39 @@
+"""The sums of the Gram kernels' partial tiles over their row chunks, at the
+chunk counts where the summation kernel's rounds of 128 chunks begin and end,
+against numpy.
+
+A thin Gram has one row chunk per 1,024 rows up to 512 chunks.  Each entry is
+a chain of at most 4 row products per thread and chunk, 8 levels of sums in
+the workgroup and the sum over at most 512 chunks, each step rounding once,
+so its error is below 530 units of roundoff of sum |x| |y|.
+"""
+import ctypes as C
+
+import numpy as np
+import pytest
+
+from gcge_amd import abi, problems as P
+from gcge_amd.solver import DeviceMatrix, HipTable
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.mark.parametrize("chunks", [1, 2, 16, 127, 128, 129, 256, 511])
+@pytest.mark.parametrize("m,n", [(1, 1), (40, 1), (3, 9)])
+def test_chunk_sums(hip, chunks, m, n):
+    rows = 1024 * chunks - (chunks * 37) % 500
+    rng = np.random.default_rng([chunks, m, n])
+    table = HipTable()
+    mat = DeviceMatrix(P.diagonal_ccs(np.ones(rows)))
+    x, y = rng.standard_normal((rows, m)), rng.standard_normal((rows, n))
+    hx, hy = table.create_multivec(m, mat), table.create_multivec(n, mat)
+    table.upload(hx, x)
+    table.upload(hy, y)
+    ip = np.full((m + 2, n), 7.0, order="F")  # rows past m stay as they are
+    table.slot("MultiVecInnerProd")(b"N", hx, hy, 0, (C.c_int * 2)(0, 0), (C.c_int * 2)(m, n),
+                                    ip.ctypes.data_as(abi.c_dbl_p), m + 2, table.ops)
+    table.destroy_multivec(hx, m)
+    table.destroy_multivec(hy, n)
+    bound = 530 * np.finfo(float).eps * (np.abs(x).T @ np.abs(y))
+    assert np.all(np.abs(ip[:m] - x.T @ y) <= bound)
+    assert np.all(ip[m:] == 7.0)
