@@ -442,13 +442,22 @@ __global__ __launch_bounds__(64) void k_sum_partials(int nparts,
 
 // ---------------------------------------------------------------------
 // Thin Gram blocks, G (m x n) = X^T Y with n <= 8 (the one-column products
-// of the column-by-column orthogonalization): a GEMV-like stream, one
-// thread per row, MT = 64 / NB columns of X per workgroup and all n columns
-// of Y in registers; X and Y are each read once per column tile.  Partial
-// sums per row chunk are combined by sum_chunks in a fixed order.
+// of the column-by-column orthogonalization): a stream bound by HBM.  A
+// workgroup takes kThinM columns of X, all n columns of Y and one chunk of
+// rows, one row per thread at a time; every load of a row is issued before
+// its first use (columns past m or n read the last one, and their sums are
+// dropped), and the kThinM NB sums of a wavefront are reduced together by
+// halving (10 exchanges for 8 sums).  Partial sums per row chunk are
+// combined by sum_chunks in a fixed order.  The form with 64 / NB columns
+// per workgroup and a test around each column's load had one load in flight
+// and 384 exchanges per wavefront whatever m was: 512 K rows by 1 to 40
+// columns, one column each, 54 us on average, now 17 (5 TB/s).  Rows, chunks
+// and the order of every sum are as there, so the bits are.
 // ---------------------------------------------------------------------
+constexpr int kThinM = 8;
+
 struct ThinPlan {
-    int nb, mt, mtiles, nchunk;
+    int nb, mtiles, nchunk;
     int64_t rows_per_chunk;
 };
 
@@ -456,19 +465,43 @@ ThinPlan thin_plan(int64_t nrows, int m, int n)
 {
     ThinPlan p;
     p.nb = n <= 1 ? 1 : n <= 2 ? 2 : n <= 4 ? 4 : 8;
-    p.mt = 64 / p.nb;
-    p.mtiles = (m + p.mt - 1) / p.mt;
-    // a few long-lived workgroups per CU: the register accumulators are
-    // reduced once per workgroup, so each should stream many rows (at most
-    // 512 in total, so no straggler round)
-    int64_t want = 512 / p.mtiles;
-    int64_t cap = (nrows + 1023) / 1024;  // at least 1024 rows per chunk
+    p.mtiles = (m + kThinM - 1) / kThinM;
+    // at most 512 chunks per 64 sums a row, at least 1024 rows per chunk:
+    // each workgroup streams many rows per reduction
+    const int64_t groups = ((int64_t)m * p.nb + 63) / 64;
+    int64_t want = 512 / groups;
+    int64_t cap = (nrows + 1023) / 1024;
     int64_t nc = want < cap ? want : cap;
     if (nc < 1) nc = 1;
     p.rows_per_chunk = (nrows + nc - 1) / nc;
     p.nchunk = (int)((nrows + p.rows_per_chunk - 1) / p.rows_per_chunk);
     if (p.nchunk < 1) p.nchunk = 1;
     return p;
+}
+
+// Sums of M values per lane over the wavefront, each by the pairs of
+// wave_sum (lanes 32 apart, then 16, ...): the steps of the first log2(M)
+// levels keep half the values on each side.  Returns the sum of value
+// `which` (set to this lane's), valid on every lane.
+template <int M>
+__device__ __forceinline__ double wave_sums(double (&v)[M], int &which)
+{
+    const int lane = threadIdx.x & 63;
+    which = 0;
+#pragma unroll
+    for (int h = M / 2, o = 32; h > 0; h >>= 1, o >>= 1) {
+        const bool up = (lane & o) != 0;
+#pragma unroll
+        for (int i = 0; i < h; ++i) {
+            const double keep = up ? v[i + h] : v[i], give = up ? v[i] : v[i + h];
+            v[i] = keep + __shfl_xor(give, o, 64);
+        }
+        which += up ? h : 0;
+    }
+    double s = v[0];
+#pragma unroll
+    for (int o = 32 / M; o > 0; o >>= 1) s += __shfl_xor(s, o, 64);
+    return s;
 }
 
 template <int NB>
@@ -478,45 +511,39 @@ __global__ __launch_bounds__(kWG) void k_gram_thin(int64_t nrows, int m, int n,
                                                    int64_t rows_per_chunk,
                                                    double *__restrict__ partial)
 {
-    constexpr int MT = 64 / NB;
-    __shared__ double red[kWG / 64][MT * NB];
-    const int chunk = blockIdx.x, mt = blockIdx.y;
-    const int i0 = mt * MT;
+    constexpr int M = kThinM * NB;
+    __shared__ double red[kWG / 64][M];
+    const int chunk = blockIdx.x, i0 = blockIdx.y * kThinM;
     const int64_t rbeg = (int64_t)chunk * rows_per_chunk;
     int64_t rend = rbeg + rows_per_chunk;
     if (rend > nrows) rend = nrows;
-    double acc[MT][NB];
+    double acc[M];
 #pragma unroll
-    for (int i = 0; i < MT; ++i)
-#pragma unroll
-        for (int q = 0; q < NB; ++q) acc[i][q] = 0.0;
+    for (int e = 0; e < M; ++e) acc[e] = 0.0;
+#pragma unroll 2
     for (int64_t r = rbeg + threadIdx.x; r < rend; r += kWG) {
-        double yv[NB];
+        double xv[kThinM], yv[NB];
 #pragma unroll
-        for (int q = 0; q < NB; ++q) yv[q] = (q < n) ? Y[r + (int64_t)q * ldy] : 0.0;
+        for (int q = 0; q < NB; ++q) yv[q] = Y[r + (int64_t)(q < n ? q : n - 1) * ldy];
 #pragma unroll
-        for (int i = 0; i < MT; ++i) {
-            if (i0 + i < m) {
-                const double xv = X[r + (int64_t)(i0 + i) * ldx];
+        for (int i = 0; i < kThinM; ++i)
+            xv[i] = X[r + (int64_t)(i0 + i < m ? i0 + i : m - 1) * ldx];
 #pragma unroll
-                for (int q = 0; q < NB; ++q) acc[i][q] += xv * yv[q];
-            }
-        }
+        for (int i = 0; i < kThinM; ++i)
+#pragma unroll
+            for (int q = 0; q < NB; ++q) acc[i * NB + q] += xv[i] * yv[q];
     }
-    const int wv = threadIdx.x >> 6, ln = threadIdx.x & 63;
-#pragma unroll
-    for (int i = 0; i < MT; ++i)
-#pragma unroll
-        for (int q = 0; q < NB; ++q) {
-            const double v = wave_sum(acc[i][q]);
-            if (ln == 0) red[wv][i * NB + q] = v;
-        }
+    int which;
+    const double s = wave_sums<M>(acc, which);
+    const int wv = threadIdx.x >> 6;
+    // the lanes that share a value hold the same sum
+    if ((threadIdx.x & (64 / M - 1)) == 0) red[wv][which] = s;
     __syncthreads();
-    for (int e = threadIdx.x; e < MT * NB; e += kWG) {
-        double s = 0.0;
+    if (threadIdx.x < M) {
+        double t = 0.0;
 #pragma unroll
-        for (int w = 0; w < kWG / 64; ++w) s += red[w][e];
-        partial[((int64_t)chunk * gridDim.y + mt) * (MT * NB) + e] = s;
+        for (int w = 0; w < kWG / 64; ++w) t += red[w][threadIdx.x];
+        partial[((int64_t)chunk * gridDim.y + blockIdx.y) * M + threadIdx.x] = t;
     }
 }
 
@@ -586,7 +613,7 @@ void gram_thin(int64_t nrows, int m, int n, const double *X, int64_t ldx, const 
     case 4: k_gram_thin<4><<<g, kWG, 0, s>>>(nrows, m, n, X, ldx, Y, ldy, p.rows_per_chunk, partial); break;
     default: k_gram_thin<8><<<g, kWG, 0, s>>>(nrows, m, n, X, ldx, Y, ldy, p.rows_per_chunk, partial); break;
     }
-    sum_chunks(m, n, p.mtiles, 1, p.mt, p.nb, p.nchunk, partial, G, ldg, transposed, s);
+    sum_chunks(m, n, p.mtiles, 1, kThinM, p.nb, p.nchunk, partial, G, ldg, transposed, s);
 }
 
 // ---------------------------------------------------------------------
@@ -750,7 +777,7 @@ static bool gram_is_thin(int m, int n) { return m <= 8 || n <= 8; }
 static int64_t thin_scratch(int64_t nrows, int m, int n)
 {
     ThinPlan p = (n <= 8) ? thin_plan(nrows, m, n) : thin_plan(nrows, n, m);
-    return (int64_t)p.nchunk * p.mtiles * p.mt * p.nb;
+    return (int64_t)p.nchunk * p.mtiles * kThinM * p.nb;
 }
 
 GramPlan gram_plan(int64_t nrows, int m, int n, bool lower_only)

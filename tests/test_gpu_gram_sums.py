@@ -18,11 +18,8 @@ from gcge_amd.solver import DeviceMatrix, HipTable
 pytestmark = pytest.mark.gpu
 
 
-@pytest.mark.parametrize("chunks", [1, 2, 16, 127, 128, 129, 256, 511])
-@pytest.mark.parametrize("m,n", [(1, 1), (40, 1), (3, 9)])
-def test_chunk_sums(hip, chunks, m, n):
-    rows = 1024 * chunks - (chunks * 37) % 500
-    rng = np.random.default_rng([chunks, m, n])
+def check(rows, m, n):
+    rng = np.random.default_rng([rows, m, n])
     table = HipTable()
     mat = DeviceMatrix(P.diagonal_ccs(np.ones(rows)))
     x, y = rng.standard_normal((rows, m)), rng.standard_normal((rows, n))
@@ -37,3 +34,16 @@ def test_chunk_sums(hip, chunks, m, n):
     bound = 530 * np.finfo(float).eps * (np.abs(x).T @ np.abs(y))
     assert np.all(np.abs(ip[:m] - x.T @ y) <= bound)
     assert np.all(ip[m:] == 7.0)
+
+
+@pytest.mark.parametrize("chunks", [1, 2, 16, 127, 128, 129, 256, 511])
+@pytest.mark.parametrize("m,n", [(1, 1), (40, 1), (3, 9)])
+def test_chunk_sums(hip, chunks, m, n):
+    check(1024 * chunks - (chunks * 37) % 500, m, n)
+
+
+@pytest.mark.parametrize("rows", [1, 63, 300, 1025, 4099])
+@pytest.mark.parametrize("m,n", [(1, 2), (7, 3), (8, 4), (9, 5), (17, 8), (65, 1), (2, 33)])
+def test_thin_tiles(hip, rows, m, n):
+    """Column tiles of 8 with remainders on both sides, thin on either side."""
+    check(rows, m, n)
