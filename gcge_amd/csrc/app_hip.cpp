@@ -1189,8 +1189,10 @@ void *HIPCCS_Create(const gcge_ccs_mat *host, int flags)
         M->bytes += (int64_t)(sizeof(float) * v32.size());
     }
     detect_plane(S, c.stream);
-    if (!(flags & GCGE_HIP_MAT_GENERAL))
+    if (!(flags & GCGE_HIP_MAT_GENERAL)) {
         S.stencil_n = detect_stencil7(host, &S.stencil_d, &S.stencil_o);
+        detect_grid27(S, c.stream);
+    }
     return M;
 }
 

@@ -343,6 +343,8 @@ void *HIPCCS_CreateGrid(const gcge_grid_op *op, int flags)
         S.stencil_d = a.dval;
         S.stencil_o = a.oval;
     }
+    if (form == kDiff27 && !(flags & GCGE_HIP_MAT_GENERAL) && n >= 4 && n <= kGrid27MaxN)
+        S.grid27_n = (int)n;
     return M;
 }
 

@@ -28,6 +28,10 @@ struct SellMat {
     // (stencil.hip), 0 otherwise.
     int stencil_n = 0;
     double stencil_d = 0.0, stencil_o = 0.0;
+    // 27-point operator on a grid27_n^3 grid (any values, the entries of each
+    // row its in-grid neighbours in ascending order), whose products take the
+    // neighbours by grid position (grid27.hip); 0 otherwise.
+    int grid27_n = 0;
     uint64_t structure_hash = 0;   // of the slice widths, to match A and B
     int64_t *slice_ptr = nullptr;  // nslices + 1
     int *col = nullptr;
@@ -62,6 +66,22 @@ bool stencil_residual(const SellMat &A, const SellMat &B, const double *X, int64
 int stencil_pw_parts(const SellMat &A, int nt_bound);
 void stencil_pw(const SellMat &A, const int *tiles, const int *ntact_p, int nt_bound,
                 const float *P, float *W, float *partial, hipStream_t s);
+// Largest grid side of the 27-point kernels (32-bit byte offsets into a
+// column and into an 8-column FP32 tile, with room to point past their end).
+constexpr int kGrid27MaxN = 256;
+// Sets A.grid27_n from A's device arrays (stream-ordered, waits for the
+// stream).
+void detect_grid27(SellMat &A, hipStream_t s);
+// The 27-point forms of spmm, of the FP32 BlockPCG's product over the listed
+// tiles (one partial p.w sum per 256 rows, as the SELL kernel's) and of its
+// FP64 residual in tiles: false, nothing done, when A.grid27_n is 0; the same
+// bits as the SELL kernels.
+bool spmm_grid27(const SellMat &A, const double *X, int64_t ldx, double *Y, int64_t ldy,
+                 int ncols, hipStream_t s);
+bool grid27_pw(const SellMat &A, const int *tiles, const int *ntact_p, const float *P, float *W,
+               float *partial, hipStream_t s);
+bool grid27_resid(const SellMat &A, int nc, const double *B, int64_t ldb, const double *X,
+                  int64_t ldx, float *R, float *partial, hipStream_t s);
 // Y[:, c] = A X[:, c], c < ncols.
 void spmm(const SellMat &A, const double *X, int64_t ldx, double *Y, int64_t ldy,
           int ncols, hipStream_t s);

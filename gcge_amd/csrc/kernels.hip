@@ -17,6 +17,7 @@
 #include "app_hip_internal.h"
 #include "kernels.h"
 #include "sell_rows.h"
+#include "tile8.h"
 #include "tuner.h"
 
 namespace gcge {
@@ -479,31 +480,6 @@ ThinPlan thin_plan(int64_t nrows, int m, int n)
     return p;
 }
 
-// Sums of M values per lane over the wavefront, each by the pairs of
-// wave_sum (lanes 32 apart, then 16, ...): the steps of the first log2(M)
-// levels keep half the values on each side.  Returns the sum of value
-// `which` (set to this lane's), valid on every lane.
-template <int M>
-__device__ __forceinline__ double wave_sums(double (&v)[M], int &which)
-{
-    const int lane = threadIdx.x & 63;
-    which = 0;
-#pragma unroll
-    for (int h = M / 2, o = 32; h > 0; h >>= 1, o >>= 1) {
-        const bool up = (lane & o) != 0;
-#pragma unroll
-        for (int i = 0; i < h; ++i) {
-            const double keep = up ? v[i + h] : v[i], give = up ? v[i] : v[i + h];
-            v[i] = keep + __shfl_xor(give, o, 64);
-        }
-        which += up ? h : 0;
-    }
-    double s = v[0];
-#pragma unroll
-    for (int o = 32 / M; o > 0; o >>= 1) s += __shfl_xor(s, o, 64);
-    return s;
-}
-
 template <int NB>
 __global__ __launch_bounds__(kWG) void k_gram_thin(int64_t nrows, int m, int n,
                                                    const double *__restrict__ X, int64_t ldx,
@@ -720,6 +696,7 @@ void spmm(const SellMat &A, const double *X, int64_t ldx, double *Y, int64_t ldy
           hipStream_t s)
 {
     if (spmm_stencil(A, X, ldx, Y, ldy, ncols, s)) return;
+    if (spmm_grid27(A, X, ldx, Y, ldy, ncols, s)) return;
     launch_spmm<double>(A, A.val, X, ldx, Y, ldy, ncols, s);
 }
 

@@ -47,72 +47,14 @@
 #include "gcge_hip.h"
 #include "kernels.h"
 #include "sell_rows.h"
+#include "tile8.h"
 #include "tuner.h"
 
 namespace gcge {
 namespace {
 
 constexpr int kWG = 256;
-constexpr int kC = 8;      // columns per interleaved tile
 constexpr int kCheck = 4;  // inner iterations between reads of the active count
-
-struct alignas(32) f8 {
-    float v[kC];
-};
-
-__device__ __forceinline__ float wave_sum(float v)
-{
-#pragma unroll
-    for (int o = 32; o > 0; o >>= 1) v += __shfl_xor(v, o, 64);
-    return v;
-}
-
-// Sum over the workgroup of kC per-thread values; result in red[4*kC + t].
-__device__ __forceinline__ void block_sum8(const float (&v)[kC], float *red)
-{
-    const int wv = threadIdx.x >> 6, ln = threadIdx.x & 63;
-#pragma unroll
-    for (int t = 0; t < kC; ++t) {
-        const float s = wave_sum(v[t]);
-        if (ln == 0) red[wv * kC + t] = s;
-    }
-    __syncthreads();
-    if (threadIdx.x < kC) {
-        float s = 0.f;
-#pragma unroll
-        for (int k = 0; k < kWG / 64; ++k) s += red[k * kC + threadIdx.x];
-        red[kWG / 64 * kC + threadIdx.x] = s;
-    }
-    __syncthreads();
-}
-
-__device__ __forceinline__ f8 load8(const float *p)
-{
-    return *reinterpret_cast<const f8 *>(p);
-}
-
-__device__ __forceinline__ void store8(float *p, const f8 &x)
-{
-    *reinterpret_cast<f8 *>(p) = x;
-}
-
-typedef float f4v __attribute__((ext_vector_type(4)));
-
-// load8 through a buffer resource at a byte offset (two 16-byte loads).
-// The loaded vectors are bit-cast whole: a bit cast of one element of the
-// integer vector reads the vector's first element for every index.
-__device__ __forceinline__ f8 buffer_load8(__amdgpu_buffer_rsrc_t r, uint32_t off)
-{
-    const f4v a = __builtin_bit_cast(f4v, __builtin_amdgcn_raw_buffer_load_b128(r, off, 0, 0));
-    const f4v b = __builtin_bit_cast(f4v, __builtin_amdgcn_raw_buffer_load_b128(r, off + 16, 0, 0));
-    f8 x;
-#pragma unroll
-    for (int i = 0; i < 4; ++i) {
-        x.v[i] = a[i];
-        x.v[4 + i] = b[i];
-    }
-    return x;
-}
 
 // Residual of the FP64 system, rounded to FP32, for every column c < nc:
 // R[c] = fl32(b[:, c] - (A + sigma B) x[:, c]) with the products in FP64
@@ -1128,9 +1070,12 @@ void pcg32_solve(void *matA, void **mv_b, void **mv_x, int *start, int *end, OPS
     if (pch < 0 || pch > 1) pch = 0;
     bool xc = pch == 1;
     k_zero_tiles<<<dim3(nblk_row, ntile), kWG, 0, st>>>(n, S.x);
-    {
-        const double *b64 = Bv->d + (int64_t)start[0] * Bv->ldd;
-        const double *x64 = Xv->d + (int64_t)start[1] * Xv->ldd;
+    const double *b64 = Bv->d + (int64_t)start[0] * Bv->ldd;
+    const double *x64 = Xv->d + (int64_t)start[1] * Xv->ldd;
+    // a 27-point grid operator without shift takes its neighbours by grid
+    // position (grid27.hip; same sums, same bits)
+    const bool grid27 = A->sell.grid27_n > 0 && sigma == 0.f;
+    if (!grid27 || !grid27_resid(A->sell, nc, b64, Bv->ldd, x64, Xv->ldd, S.r, S.partial, st)) {
         const double *vB = (Bs != &A->sell) ? Bs->val : nullptr;
 #define RESID(W, SH, XC)                                                                      \
     k_resid64<W, SH, XC><<<nblk_row, kWG, 0, st>>>(n, A->sell.slice_ptr, A->sell.col,            \
@@ -1234,6 +1179,7 @@ void pcg32_solve(void *matA, void **mv_b, void **mv_x, int *start, int *end, OPS
             stencil_pw(A->sell, tl, nt_p, nt_bound, S.p, S.w, S.partial, st);
             return;
         }
+        if (grid27 && grid27_pw(A->sell, tl, nt_p, S.p, S.w, S.partial, st)) return;
 #define SPMM_PW(W, TWO, XC)                                                                   \
     k_spmm_pw<W, TWO, XC><<<nblk_row, kWG, 0, st>>>(n, A->sell.slice_ptr, A->sell.col,        \
                                                     A->sell.val32, Bs->col, vB, sigma, tl,     \
@@ -1253,7 +1199,7 @@ void pcg32_solve(void *matA, void **mv_b, void **mv_x, int *start, int *end, OPS
         }
 #undef SPMM_PW
     };
-    if (tune_pw && ntact > 0 && sparts == 0) {
+    if (tune_pw && ntact > 0 && sparts == 0 && !grid27) {
         // the tile list and count are set; p is written by the first
         // iteration before it is read, and w and the partials are
         // overwritten by every launch, so the timing runs leave no trace
