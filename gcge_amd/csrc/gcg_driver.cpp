@@ -36,6 +36,11 @@ int64_t pcg32_iterations(OPS *ops);
 // operators of one grid (false otherwise); app_hip.cpp.
 bool hip_stencil_residual(OPS *ops, void *A, void *B, void **x, int sx, int nc,
                           const double *lam, void **r, int sr);
+// A BlockPCG step's column updates in one launch each when ops is the HIP
+// table (false otherwise); app_hip.cpp.
+bool hip_cg_p(OPS *ops, void **r, void **p, const int *cols, const double *beta, int n);
+bool hip_cg_xr(OPS *ops, void **p, void **w, void **x, int x0, void **r, const int *cols,
+               const double *alpha, int n, double *rr);
 int hip_cholqr_pass(OPS *ops, void **x, int sx, int n, void *B, void **mv_ws, double zero_tol,
                     double rel_tol);
 int hip_orth_coef_comb(OPS *ops, double *Z, int n, int sp, int np, double zero_tol,
@@ -394,7 +399,7 @@ void block_pcg(Solver &S, void **mv_b, void **mv_x, int *start_bx, int *end_bx)
     const int n0 = end_bx[0] - start_bx[0];
     const double rate = S.cg_rate, tol = S.cg_tol;
     std::vector<double> norm_b((size_t)n0, 1.0), rho1((size_t)n0), rho2((size_t)n0),
-        pTw((size_t)n0), init_res((size_t)n0), last_res((size_t)n0);
+        pTw((size_t)n0), init_res((size_t)n0), last_res((size_t)n0), coef((size_t)n0);
     std::vector<int> unconv((size_t)n0), block((size_t)n0 + 1);
     int s[2], e[2];
     if (S.cg_tol_type == "rel") {
@@ -429,37 +434,44 @@ void block_pcg(Solver &S, void **mv_b, void **mv_x, int *start_bx, int *end_bx)
             if (unconv[i] - unconv[i - 1] > 1) block[nblock++] = i;
         block[nblock] = nu;
         double *dst = pTw.data();
-        for (int b = 0; b < nblock; ++b) {
-            const int len = block[b + 1] - block[b];
-            for (int c = block[b]; c < block[b + 1]; ++c) {
-                const double beta = (niter == 0) ? 0.0 : rho2[c] / rho1[c];
+        for (int c = 0; c < nu; ++c) coef[c] = (niter == 0) ? 0.0 : rho2[c] / rho1[c];
+        if (!gcge::hip_cg_p(ops, r, p, unconv.data(), coef.data(), nu)) {
+            for (int c = 0; c < nu; ++c) {
                 s[0] = unconv[c]; e[0] = unconv[c] + 1;
                 s[1] = unconv[c]; e[1] = unconv[c] + 1;
-                ops->MultiVecAxpby(1.0, r, beta, p, s, e, ops);
+                ops->MultiVecAxpby(1.0, r, coef[c], p, s, e, ops);
             }
+        }
+        for (int b = 0; b < nblock; ++b) {
+            const int len = block[b + 1] - block[b];
             s[0] = unconv[block[b]]; e[0] = unconv[block[b + 1] - 1] + 1;
             s[1] = s[0]; e[1] = e[0];
             shifted_apply(S, p, w, s, e, mv_b, start_bx[0]);
             ops->MultiVecLocalInnerProd('D', p, w, 0, s, e, dst, 1, ops);
             dst += len;
         }
-        for (int i = 0; i < nu; ++i) rho1[i] = rho2[i];
-        dst = rho2.data();
-        for (int b = 0; b < nblock; ++b) {
-            const int len = block[b + 1] - block[b];
-            for (int c = block[b]; c < block[b + 1]; ++c) {
-                const double alpha = rho2[c] / pTw[c];
-                s[0] = unconv[c]; e[0] = unconv[c] + 1;
-                s[1] = start_bx[1] + unconv[c]; e[1] = s[1] + 1;
-                ops->MultiVecAxpby(alpha, p, 1.0, mv_x, s, e, ops);
-                s[0] = unconv[c]; e[0] = unconv[c] + 1;
-                s[1] = unconv[c]; e[1] = unconv[c] + 1;
-                ops->MultiVecAxpby(-alpha, w, 1.0, r, s, e, ops);
+        for (int i = 0; i < nu; ++i) {
+            rho1[i] = rho2[i];
+            coef[i] = rho2[i] / pTw[i];
+        }
+        if (!gcge::hip_cg_xr(ops, p, w, mv_x, start_bx[1], r, unconv.data(), coef.data(), nu,
+                             rho2.data())) {
+            dst = rho2.data();
+            for (int b = 0; b < nblock; ++b) {
+                const int len = block[b + 1] - block[b];
+                for (int c = block[b]; c < block[b + 1]; ++c) {
+                    s[0] = unconv[c]; e[0] = unconv[c] + 1;
+                    s[1] = start_bx[1] + unconv[c]; e[1] = s[1] + 1;
+                    ops->MultiVecAxpby(coef[c], p, 1.0, mv_x, s, e, ops);
+                    s[0] = unconv[c]; e[0] = unconv[c] + 1;
+                    s[1] = unconv[c]; e[1] = unconv[c] + 1;
+                    ops->MultiVecAxpby(-coef[c], w, 1.0, r, s, e, ops);
+                }
+                s[0] = unconv[block[b]]; e[0] = unconv[block[b + 1] - 1] + 1;
+                s[1] = s[0]; e[1] = e[0];
+                ops->MultiVecLocalInnerProd('D', r, r, 0, s, e, dst, 1, ops);
+                dst += len;
             }
-            s[0] = unconv[block[b]]; e[0] = unconv[block[b + 1] - 1] + 1;
-            s[1] = s[0]; e[1] = e[0];
-            ops->MultiVecLocalInnerProd('D', r, r, 0, s, e, dst, 1, ops);
-            dst += len;
         }
         for (int i = 0; i < nu; ++i) last_res[unconv[i]] = std::sqrt(rho2[i]);
         const int pre = nu;

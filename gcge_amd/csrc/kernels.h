@@ -105,6 +105,27 @@ void sum_chunks(int m, int n, int tm, int tn, int TM, int TN, int nchunk, const 
                 double *G, int ldg, bool transposed, hipStream_t s);
 void col_dots(int64_t nrows, int ncols, const double *X, int64_t ldx, const double *Y,
               int64_t ldy, double *out, double *partial, hipStream_t s);
+// One BlockPCG step on up to kCgCols listed columns, each column with its own
+// coefficient (the arithmetic of axpby):
+//   cg_p:  P[:, col] = R[:, col] + a P[:, col] (P is not read where a is 0)
+//   cg_xr: X[:, x0 + col] += a P[:, col], R[:, col] -= a W[:, col]
+// and cg_xr_dots the latter with out[k] = R[:, col[k]] . R[:, col[k]], by the
+// sums of col_dots (partial: dots_scratch(k) doubles).
+constexpr int kCgCols = 64;
+struct CgCols {
+    int n = 0;
+    int col[kCgCols];
+    double a[kCgCols];
+};
+void cg_p(int64_t nrows, const CgCols &c, const double *R, int64_t ldr, double *P, int64_t ldp,
+          hipStream_t s);
+void cg_xr(int64_t nrows, const CgCols &c, const double *P, int64_t ldp, const double *W,
+           int64_t ldw, double *X, int64_t ldx, double *R, int64_t ldr, hipStream_t s);
+void cg_xr_dots(int64_t nrows, const CgCols &c, const double *P, int64_t ldp, const double *W,
+                int64_t ldw, double *X, int64_t ldx, double *R, int64_t ldr, double *out,
+                double *partial, hipStream_t s);
+// Whether the fused dots fill the device as the separate updates do.
+bool cg_fuse_dots(int64_t nrows, int ncols);
 // G (m x n, ldg) = X^T Y with X: nrows x m, Y: nrows x n.  lower_only
 // computes only entries with row >= col (the 'S' case).  The plan fixes
 // the kernel, its row chunking and the doubles of partial-sum scratch it
@@ -125,7 +146,8 @@ GramPlan gram_plan(int64_t nrows, int m, int n, bool lower_only);
 GramPlan gram_plan_bounded(int64_t nrows, int m, int n, bool lower_only, int64_t max_scratch);
 void gram(const GramPlan &p, int64_t nrows, int m, int n, const double *X, int64_t ldx,
           const double *Y, int64_t ldy, double *G, int ldg, bool lower_only, double *partial,
-          hipStream_t s);
+          hipStream_t s, bool rowmajor = false);
+// (rowmajor: G[i ldg + j])
 // Y (nrows x n) = X (nrows x m) C (m x n) + Y diag(beta), with C given
 // transposed and k-major: Ct[k * ldct + j] = C[k][j] (device).
 // beta_mode: 0 overwrite, 1 scalar beta_scalar, 2 per-column beta (device).
@@ -141,8 +163,8 @@ int64_t gram_mfma_scratch(int64_t nrows, int m, int n, int choice, int64_t max_c
 // doubles of partial sums per row chunk
 int64_t gram_mfma_chunk_doubles(int m, int n);
 void gram_mfma(int64_t nrows, int m, int n, const double *X, int64_t ldx, const double *Y,
-               int64_t ldy, double *G, int ldg, bool lower_only, int choice, int64_t max_chunks,
-               bool tune, double *partial, hipStream_t s);
+               int64_t ldy, double *G, int ldg, bool rowmajor, bool lower_only, int choice,
+               int64_t max_chunks, bool tune, double *partial, hipStream_t s);
 void lincomb_mfma(int64_t nrows, int m, int n, const double *X, int64_t ldx, const double *Ct,
                   int ldct, int beta_mode, double beta_scalar, const double *beta, double *Y,
                   int64_t ldy, hipStream_t s);

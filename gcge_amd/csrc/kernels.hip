@@ -442,6 +442,79 @@ __global__ __launch_bounds__(64) void k_sum_partials(int nparts,
 }
 
 // ---------------------------------------------------------------------
+// The column updates of a BlockPCG step, every column with its own
+// coefficient in one launch: a driver that updates its columns one by one
+// launches three kernels per column and step, 56,640 launches of 3 us in a
+// double-precision solve of 16,384 rows in blocks of 4 (311 ms, bound by
+// their launches; 132 ms with these).
+// ---------------------------------------------------------------------
+// b y + x with the product rounded, as axpby forms it for alpha = 1
+__device__ __forceinline__ double scaled_sum(double b, double y, double x)
+{
+#pragma clang fp contract(off)
+    const double t = b * y;
+    return t + x;
+}
+
+__global__ __launch_bounds__(kWG) void k_cg_p(int64_t nrows, CgCols c,
+                                              const double *__restrict__ R, int64_t ldr,
+                                              double *__restrict__ P, int64_t ldp)
+{
+    const int col = c.col[blockIdx.y];
+    const double beta = c.a[blockIdx.y];
+    const double *r = R + (int64_t)col * ldr;
+    double *p = P + (int64_t)col * ldp;
+    const int64_t r0 = (int64_t)blockIdx.x * kWG * kRowsPerThread + threadIdx.x;
+#pragma unroll
+    for (int q = 0; q < kRowsPerThread; ++q) {
+        const int64_t i = r0 + (int64_t)q * kWG;
+        if (i < nrows) {
+            p[i] = scaled_sum(beta, beta == 0.0 ? 0.0 : p[i], r[i]);
+        }
+    }
+}
+
+// DOTS: a workgroup takes the rows of col_dots' and leaves its r.r partial
+template <bool DOTS>
+__global__ __launch_bounds__(kWG) void k_cg_xr(int64_t nrows, CgCols c,
+                                               const double *__restrict__ P, int64_t ldp,
+                                               const double *__restrict__ W, int64_t ldw,
+                                               double *__restrict__ X, int64_t ldx,
+                                               double *__restrict__ R, int64_t ldr,
+                                               double *__restrict__ partial)
+{
+    const int k = blockIdx.y, col = c.col[k];
+    const double a = c.a[k];
+    const double *p = P + (int64_t)col * ldp, *w = W + (int64_t)col * ldw;
+    double *x = X + (int64_t)col * ldx, *r = R + (int64_t)col * ldr;
+    double acc = 0.0;
+    auto step = [&](int64_t i) {
+        x[i] = fma(a, p[i], x[i]);
+        const double v = fma(-a, w[i], r[i]);
+        r[i] = v;
+        acc = fma(v, v, acc);
+    };
+    if constexpr (DOTS) {
+        for (int64_t i = (int64_t)blockIdx.x * kWG + threadIdx.x; i < nrows;
+             i += (int64_t)gridDim.x * kWG)
+            step(i);
+        acc = block_sum(acc);
+        if (threadIdx.x == 0) partial[(int64_t)k * gridDim.x + blockIdx.x] = acc;
+    } else {
+        const int64_t r0 = (int64_t)blockIdx.x * kWG * kRowsPerThread + threadIdx.x;
+#pragma unroll
+        for (int q = 0; q < kRowsPerThread; ++q)
+            if (r0 + (int64_t)q * kWG < nrows) step(r0 + (int64_t)q * kWG);
+    }
+}
+
+int dots_blocks(int64_t nrows)
+{
+    int64_t nb = (nrows + kWG * 8 - 1) / (kWG * 8);
+    return (int)(nb < 1 ? 1 : nb > kDotBlocks ? kDotBlocks : nb);
+}
+
+// ---------------------------------------------------------------------
 // Thin Gram blocks, G (m x n) = X^T Y with n <= 8 (the one-column products
 // of the column-by-column orthogonalization): a stream bound by HBM.  A
 // workgroup takes kThinM columns of X, all n columns of Y and one chunk of
@@ -738,12 +811,42 @@ void col_dots(int64_t nrows, int ncols, const double *X, int64_t ldx, const doub
               int64_t ldy, double *out, double *partial, hipStream_t s)
 {
     if (ncols <= 0) return;
-    int nb = (int)((nrows + kWG * 8 - 1) / (kWG * 8));
-    if (nb < 1) nb = 1;
-    if (nb > kDotBlocks) nb = kDotBlocks;
+    const int nb = dots_blocks(nrows);
     dim3 g(nb, ncols);
     k_col_dots_partial<<<g, kWG, 0, s>>>(nrows, X, ldx, Y, ldy, partial);
     k_sum_partials<<<ncols, 64, 0, s>>>(nb, partial, out);
+}
+
+void cg_p(int64_t nrows, const CgCols &c, const double *R, int64_t ldr, double *P, int64_t ldp,
+          hipStream_t s)
+{
+    if (nrows <= 0 || c.n <= 0) return;
+    k_cg_p<<<dim3(grid1d(nrows, kRowsPerThread), c.n), kWG, 0, s>>>(nrows, c, R, ldr, P, ldp);
+}
+
+void cg_xr(int64_t nrows, const CgCols &c, const double *P, int64_t ldp, const double *W,
+           int64_t ldw, double *X, int64_t ldx, double *R, int64_t ldr, hipStream_t s)
+{
+    if (nrows <= 0 || c.n <= 0) return;
+    k_cg_xr<false><<<dim3(grid1d(nrows, kRowsPerThread), c.n), kWG, 0, s>>>(
+        nrows, c, P, ldp, W, ldw, X, ldx, R, ldr, nullptr);
+}
+
+void cg_xr_dots(int64_t nrows, const CgCols &c, const double *P, int64_t ldp, const double *W,
+                int64_t ldw, double *X, int64_t ldx, double *R, int64_t ldr, double *out,
+                double *partial, hipStream_t s)
+{
+    if (c.n <= 0) return;
+    const int nb = dots_blocks(nrows);
+    k_cg_xr<true><<<dim3(nb, c.n), kWG, 0, s>>>(nrows, c, P, ldp, W, ldw, X, ldx, R, ldr, partial);
+    k_sum_partials<<<c.n, 64, 0, s>>>(nb, partial, out);
+}
+
+// col_dots has at most 128 workgroups per column, too few for six streams of
+// a large column when there are few of them
+bool cg_fuse_dots(int64_t nrows, int ncols)
+{
+    return dots_blocks(nrows) < kDotBlocks || ncols * kDotBlocks >= 1024;
 }
 
 // Blocks with both sides above 8 go to the matrix cores; thinner ones
@@ -790,19 +893,19 @@ GramPlan gram_plan_bounded(int64_t nrows, int m, int n, bool lower_only, int64_t
 
 void gram(const GramPlan &p, int64_t nrows, int m, int n, const double *X, int64_t ldx,
           const double *Y, int64_t ldy, double *G, int ldg, bool lower_only, double *partial,
-          hipStream_t s)
+          hipStream_t s, bool rowmajor)
 {
     if (m <= 0 || n <= 0) return;
     if (!p.thin) {
-        gram_mfma(nrows, m, n, X, ldx, Y, ldy, G, ldg, lower_only, p.choice, p.max_chunks, p.tune,
-                  partial, s);
+        gram_mfma(nrows, m, n, X, ldx, Y, ldy, G, ldg, rowmajor, lower_only, p.choice, p.max_chunks,
+                  p.tune, partial, s);
         return;
     }
     // lower_only needs no special case here: the full block is computed
     if (n <= 8)
-        gram_thin(nrows, m, n, X, ldx, Y, ldy, G, ldg, false, partial, s);
+        gram_thin(nrows, m, n, X, ldx, Y, ldy, G, ldg, rowmajor, partial, s);
     else
-        gram_thin(nrows, n, m, Y, ldy, X, ldx, G, ldg, true, partial, s);
+        gram_thin(nrows, n, m, Y, ldy, X, ldx, G, ldg, !rowmajor, partial, s);
 }
 
 void lincomb(int64_t nrows, int m, int n, const double *X, int64_t ldx, const double *Ct,

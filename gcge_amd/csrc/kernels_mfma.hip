@@ -406,7 +406,7 @@ int64_t gram_mfma_scratch(int64_t nrows, int m, int n, int choice, int64_t max_c
 namespace {
 
 void launch_gram(const GramPlanM &p, int64_t nrows, int m, int n, const double *X, int64_t ldx,
-                 const double *Y, int64_t ldy, double *G, int ldg, bool lower_only,
+                 const double *Y, int64_t ldy, double *G, int ldg, bool rowmajor, bool lower_only,
                  double *partial, hipStream_t s)
 {
     const int64_t nblk = (int64_t)p.nchunk * p.tm * p.tn;
@@ -427,14 +427,14 @@ void launch_gram(const GramPlanM &p, int64_t nrows, int m, int n, const double *
     else
         GCGE_GRAM(2, 4);
 #undef GCGE_GRAM
-    sum_chunks(m, n, p.tm, p.tn, p.sh.rows(), p.sh.cols(), p.nchunk, partial, G, ldg, false, s);
+    sum_chunks(m, n, p.tm, p.tn, p.sh.rows(), p.sh.cols(), p.nchunk, partial, G, ldg, rowmajor, s);
 }
 
 }  // namespace
 
 void gram_mfma(int64_t nrows, int m, int n, const double *X, int64_t ldx, const double *Y,
-               int64_t ldy, double *G, int ldg, bool lower_only, int choice, int64_t max_chunks,
-               bool tune, double *partial, hipStream_t s)
+               int64_t ldy, double *G, int ldg, bool rowmajor, bool lower_only, int choice,
+               int64_t max_chunks, bool tune, double *partial, hipStream_t s)
 {
     if (m <= 0 || n <= 0) return;
     if (tune) {
@@ -452,7 +452,7 @@ void gram_mfma(int64_t nrows, int m, int n, const double *X, int64_t ldx, const 
         tune_run(key, kGramCands, kGramDefault,
                  [&](int i) {
                      launch_gram(plan_cand(nrows, m, n, i), nrows, m, n, X, ldx, Y, ldy, G, ldg,
-                                 lower_only, buf, s);
+                                 rowmajor, lower_only, buf, s);
                  },
                  s);
         HIPCHECK(hipStreamSynchronize(s));
@@ -460,7 +460,7 @@ void gram_mfma(int64_t nrows, int m, int n, const double *X, int64_t ldx, const 
         return;
     }
     launch_gram(plan_of(nrows, m, n, choice, max_chunks), nrows, m, n, X, ldx, Y, ldy, G, ldg,
-                lower_only, partial, s);
+                rowmajor, lower_only, partial, s);
 }
 
 void lincomb_mfma(int64_t nrows, int m, int n, const double *X, int64_t ldx, const double *Ct,
