@@ -614,17 +614,19 @@ void h_MultiVecAxpby(double alpha, void **x, double beta, void **y, int *start, 
 }
 
 // Whether X[:, nr] C + Y diag(beta) (nc destination columns) runs as the
-// library GEMM: from 448 Ki rows with at least 100 source and 100
-// destination columns and no per-column beta (X C + beta Y is a plain
-// GEMM; 47-66 TFLOP/s against 37-53 for the matrix-core kernel at 0.5-4 M
-// rows, 150-460 source and 100-220 destination columns); otherwise the
-// matrix-core kernel (equal at 262,144-373,248 rows or 320 destination
-// columns, faster below; 35 against 23 TFLOP/s for 40 destination columns
-// at 4 M rows, whose 128-wide tiles the library fills to a third).
+// library GEMM instead of the matrix-core kernel (no per-column beta: a
+// plain GEMM then).  Both reach 62-67 TFLOP/s of what they multiply; the
+// library's tiles are 128 columns wide, the kernel's a multiple of 16, so the
+// library is taken where its tiles hold no more padding -- 120 columns of 460
+// at 2 M rows: 3.70 ms against 3.97 -- and the kernel elsewhere (141 columns
+// of 300 at 1 M rows: 2.59 against 1.54 ms; 220 of 460 at 2 M rows: 7.35
+// against 6.70); below 448 Ki rows or 100 source columns the kernel ties or
+// is faster.
 bool lincomb_library(const MV *X, const MV *Y, int nr, int nc, bool per_column_beta)
 {
-    return Y->nrows >= (int64_t(448) << 10) && nr >= 100 && nc >= 100 && !per_column_beta &&
-           Y->nrows <= INT32_MAX && X->ldd <= INT32_MAX && Y->ldd <= INT32_MAX;
+    return Y->nrows >= (int64_t(448) << 10) && nr >= 100 && (nc + 15) / 16 % 8 == 0 &&
+           !per_column_beta && Y->nrows <= INT32_MAX && X->ldd <= INT32_MAX &&
+           Y->ldd <= INT32_MAX;
 }
 
 // Y (nrows x nc) = X (nrows x nr) C + Y diag(beta) with C on the device:

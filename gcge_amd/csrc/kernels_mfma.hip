@@ -9,9 +9,11 @@
 // tests/test_gpu_slots.py).
 #include <hip/hip_runtime.h>
 #include <cstdint>
+#include <type_traits>
 
 #include "app_hip_internal.h"
 #include "kernels.h"
+#include "sell_rows.h"
 #include "tuner.h"
 
 namespace gcge {
@@ -254,124 +256,188 @@ TuneKey gram_key(int64_t nrows, int m, int n, bool lower_only)
 
 // ---------------------------------------------------------------------
 // LinearComb: Y (nrows x n) = X (nrows x m) C (m x n) + Y diag(beta),
-// evaluated as Y^T = C^T X^T.  A wave owns 64 rows x 64 columns of Y
-// (4 x 4 MFMA tiles): per step of 4 k it takes four X operands (lane l
-// reads X[i + l%16, k + l/16], 128-byte row segments straight from HBM)
-// and four C^T operands (from L1/L2: C is small) and issues 16 MFMAs, so
-// each operand feeds four matrix-core instructions.  Operands sit in a
-// ring of kRing one-step buffers: the loads for step s + kRing - 1 are
-// issued before the MFMAs of step s, and at 224-246 registers two waves share
-// each SIMD, so HBM latency hides behind the other wave's MFMAs.  The
-// accumulator holds 16 consecutive rows of one column per lane group, so
-// the stores are contiguous.  Ct is C^T packed k-major: Ct[k * ldct + j].
-// A workgroup (4 waves) covers 256 rows; consecutive workgroups on one XCD
-// take the column tiles of the same rows.
+// evaluated as Y^T = C^T X^T.  A workgroup of four waves owns 128 R2 rows by
+// 16 NB columns of Y, a wave 32 R2 rows of it (2 R2 x NB MFMA tiles).  Ct is
+// C^T packed k-major: Ct[k * ldct + j].
+//
+// X is streamed from HBM into the MFMA operand registers: a lane reads two
+// consecutive rows of a column at once, the even row for one MFMA tile and
+// the odd one for another, so a step of 4 k takes R2 16-byte loads per lane;
+// they are issued 8 steps ahead (a ring of 8).  C goes through LDS, 16 k at a
+// time and double buffered, shared by the four waves (one barrier per 16 k;
+// rows padded so that the operand reads cover the banks once).
+//
+// Bound by the matrix cores for wide blocks, by HBM for narrow ones.  Streaming
+// both operands from HBM and L2 with 8-byte loads (64 x 64 tiles per wave, as
+// before) kept the vector L1 busy more than half the time, and tiles of 64
+// columns, like the 128-wide ones of the library's GEMM, multiply padding:
+// 300 -> 141 columns at 1.03 M rows took the library 2.59 ms and the old
+// kernel 1.84 at best, now 1.54 (58 TF/s); 460 -> 220 at 2 M rows 7.35 and
+// 7.81, now 6.70; 200 -> 100 at 531 K rows 0.64 and 0.59, now 0.455; at 216 K
+// rows 0.255 before, now 0.200; 200 -> 40 at 1.4 M rows 0.66, now 0.57.
 // ---------------------------------------------------------------------
-// Ring depth by row count: over 2 M rows a 5-step ring ties with 4 without
-// beta and is 2-8 % faster with it (m = 220-460); up to 65,536 rows, where
-// launches are latency-bound, 5 steps are 1-15 % slower, so smaller
-// problems keep 4.
-constexpr int64_t kRingDeepRows = int64_t(1) << 18;
+typedef double d2 __attribute__((ext_vector_type(2)));
+typedef double d2u __attribute__((ext_vector_type(2), aligned(8)));
 
-// NB: 16-column MFMA tiles per wave (4, a 64-column tile, unless the
-// block is narrower: 40 destination columns run 48 wide instead of 64).
-template <int BM, int kRing, int NB>
-__global__ __launch_bounds__(kWG) void k_lincomb_mfma(
+constexpr int kLcK = 16;            // k per LDS chunk
+constexpr int kLcSteps = kLcK / 4;  // its steps, all of whose X loads are in flight
+constexpr int kLcMaxNB = 9;         // 144 accumulator registers (with beta 8: no room to spare)
+// Narrow tiles take 64 rows per wave from this many workgroups on: half the
+// reads of C per row (200 -> 40 columns at 1.4 M rows: 0.61 -> 0.57 ms).
+constexpr int64_t kLcTallWg = 512;
+
+// BIG: offsets of X or C past the 32 bits of a buffer load
+template <int BM, int R2, int NB, bool BIG>
+__global__ __launch_bounds__(kWG, 2) void k_lincomb(
     int64_t nrows, int m, int n, const double *__restrict__ X, int64_t ldx,
     const double *__restrict__ Ct, int ldct, double beta_scalar,
     const double *__restrict__ beta, double *__restrict__ Y, int64_t ldy, int ntj)
 {
+    constexpr int kCols = 16 * NB;
+    constexpr int kLd = NB % 2 == 0 ? kCols + 16 : kCols;
+    __shared__ double sc[2][kLcK * kLd];
     const int64_t lb = xcd_swizzle(blockIdx.x, gridDim.x);
-    const int tj = (int)(lb % ntj);
-    const int64_t tb = lb / ntj;
+    const int j0 = (int)(lb % ntj) * kCols;
     const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
     const int li = lane & 15, lk = lane >> 4;
-    const int64_t i0 = tb * 256 + wave * 64;
-    const int j0 = tj * 16 * NB;
-    bool rok[4];
-    const double *xr[4];
+    const int64_t i0 = lb / ntj * (128 * R2) + wave * (32 * R2);
+    // the lane's row pairs (pr, pr + 1), read from rs: a pair that would pass
+    // the last row reads the one before instead
+    int64_t rs[R2];
+    bool ok0[R2], ok1[R2];
+    uint32_t xo[R2];
 #pragma unroll
-    for (int a = 0; a < 4; ++a) {
-        const int64_t row = i0 + a * 16 + li;
-        rok[a] = row < nrows;
-        xr[a] = X + (rok[a] ? row : 0);
+    for (int g = 0; g < R2; ++g) {
+        const int64_t pr = i0 + g * 32 + 2 * li;
+        int64_t r = pr < nrows - 2 ? pr : nrows - 2;
+        if (r < 0) r = 0;
+        rs[g] = r;
+        ok0[g] = pr < nrows && r == pr;
+        ok1[g] = pr < nrows && r + 1 < nrows;
+        xo[g] = (uint32_t)((r + (int64_t)lk * ldx) * 8);
     }
-    bool jok[NB];
+    d4 acc[2 * R2][NB];
 #pragma unroll
-    for (int q = 0; q < NB; ++q) jok[q] = (j0 + q * 16 + li) < n;
-    // BM (beta mode) 0: overwrite; 1: scalar beta; 2: per-column beta.  The
-    // accumulators start from Y diag(beta), read 16 at a time (a scheduling
-    // barrier after each row tile keeps the 64 loads from being in flight at
-    // once, which would double the registers and halve the occupancy)
-    d4 acc[4][NB];
-#pragma unroll
-    for (int a = 0; a < 4; ++a) {
-        // out-of-range rows and columns read a clamped in-range element and
-        // are zeroed by the select (no branch per element)
-        const int64_t rowc = rok[a] ? i0 + a * 16 + li : nrows - 1;
+    for (int g = 0; g < R2; ++g) {
 #pragma unroll
         for (int q = 0; q < NB; ++q) {
-            d4 init;
+            if (BM == 0) {
+                acc[2 * g][q] = acc[2 * g + 1][q] = d4{0.0, 0.0, 0.0, 0.0};
+                continue;
+            }
+            // Y diag(beta) first, read 8 values at a time; D = 0 * 0 + init
+            // moves them into the accumulator registers
+            d4 e, o;
 #pragma unroll
             for (int v = 0; v < 4; ++v) {
                 const int j = j0 + q * 16 + lk + 4 * v;
-                if (BM == 0) {
-                    init[v] = 0.0;
-                } else {
-                    const int jc = j < n ? j : n - 1;
-                    const double bb = BM == 2 ? beta[jc] : beta_scalar;
-                    const double y = Y[rowc + (int64_t)jc * ldy];
-                    init[v] = (rok[a] && j < n && bb != 0.0) ? bb * y : 0.0;
-                }
+                const int jc = j < n ? j : n - 1;
+                const double bb = BM == 2 ? beta[jc] : beta_scalar;
+                const double *y = Y + rs[g] + (int64_t)jc * ldy;
+                const bool use = j < n && bb != 0.0;
+                const double y0 = y[0], y1 = y[ok1[g] ? 1 : 0];
+                e[v] = use ? bb * y0 : 0.0;
+                o[v] = use ? bb * y1 : 0.0;
             }
-            // D = 0 * 0 + init moves the value into the accumulator registers
-            acc[a][q] = BM == 0 ? init : mfma(0.0, 0.0, init);
-        }
-        if (BM != 0) asm volatile("" ::: "memory");
-    }
-    // bx[b][a]: X operand of row tile a, ac[b][q]: C^T operand of column
-    // tile q, for the step held in ring buffer b; steps past m load zeros
-    double bx[kRing][4], ac[kRing][NB];
-    // one step into ring buffer B (a macro: the ring index must stay a
-    // compile-time constant for the buffers to live in registers)
-#define GCGE_LC_LOAD(B, STEP)                                                         \
-    {                                                                                 \
-        const int k_ = (STEP) * 4 + lk;                                               \
-        const bool kok_ = k_ < m;                                                     \
-        _Pragma("unroll") for (int a = 0; a < 4; ++a) bx[B][a] =                      \
-            (kok_ && rok[a]) ? xr[a][(int64_t)k_ * ldx] : 0.0;                        \
-        const double *cr_ = Ct + (int64_t)(kok_ ? k_ : 0) * ldct + j0 + li;           \
-        _Pragma("unroll") for (int q = 0; q < NB; ++q) ac[B][q] =                     \
-            (kok_ && jok[q]) ? cr_[q * 16] : 0.0;                                     \
-    }
-#pragma unroll
-    for (int b = 0; b < kRing - 1; ++b) GCGE_LC_LOAD(b, b);
-    const int nsteps = (m + 3) / 4;
-    for (int s0 = 0; s0 < nsteps; s0 += kRing) {
-#pragma unroll
-        for (int u = 0; u < kRing; ++u) {
-            // refill the buffer the previous step used
-            GCGE_LC_LOAD((u + kRing - 1) % kRing, s0 + u + kRing - 1);
-#pragma unroll
-            for (int a = 0; a < 4; ++a)
-#pragma unroll
-                for (int q = 0; q < NB; ++q) acc[a][q] = mfma(ac[u][q], bx[u][a], acc[a][q]);
+            acc[2 * g][q] = mfma(0.0, 0.0, e);
+            acc[2 * g + 1][q] = mfma(0.0, 0.0, o);
+            asm volatile("" ::: "memory");
         }
     }
-#undef GCGE_LC_LOAD
-    // lane l holds (Y^T)[j0 + q*16 + l/16 + 4v][i0 + a*16 + l%16]
+    const int nchunks = (m + kLcK - 1) / kLcK;
+    d2 ring[kLcSteps][R2];
+    // the next step's columns of X: those from m on lie past the buffer's end
+    // and read as zero, so no load is conditional and none is waited for early
+    const double *xk = X;
+    int64_t left = ((int64_t)(m - 1) * ldx + nrows) * 8;
+    int64_t xl[BIG ? R2 : 1];
+    if (BIG)
+        for (int g = 0; g < R2; ++g) xl[g] = rs[g] + (int64_t)lk * ldx;
+    int kl = lk;
+    auto load_x = [&](d2 (&to)[R2]) {
+        if constexpr (BIG) {
 #pragma unroll
-    for (int a = 0; a < 4; ++a) {
-        if (!rok[a]) continue;
-        const int64_t row = i0 + a * 16 + li;
+            for (int g = 0; g < R2; ++g) {
+                const double *p = X + (kl < m ? xl[g] : rs[g]);
+                to[g] = kl < m ? d2{p[0], p[ok1[g] ? 1 : 0]} : d2{0.0, 0.0};
+                xl[g] += 4 * ldx;
+            }
+            kl += 4;
+            return;
+        }
+        const auto rsrc = buffer_rsrc(
+            xk, left <= 0 ? 0u : left > (int64_t)UINT32_MAX ? UINT32_MAX : (uint32_t)left);
+#pragma unroll
+        for (int g = 0; g < R2; ++g)
+            to[g] = __builtin_bit_cast(d2, __builtin_amdgcn_raw_buffer_load_b128(rsrc, xo[g], 0, 0));
+        left -= 32 * ldx;
+        xk += left > 0 ? 4 * ldx : 0;
+    };
+    // C: rows from m on read as zero; a column past n holds what follows it
+    // in memory, for results that are not stored
+    const auto crsrc = buffer_rsrc(Ct, (uint32_t)(((int64_t)(m - 1) * ldct + n) * 8));
+    double cst[NB];
+    auto load_c = [&](int chunk) {
+#pragma unroll
+        for (int u = 0; u < NB; ++u) {
+            const int e = threadIdx.x + kWG * u;
+            const int k = chunk * kLcK + e / kCols, j = j0 + e % kCols;
+            if constexpr (BIG)
+                cst[u] = k < m && j < n ? Ct[(int64_t)k * ldct + j] : 0.0;
+            else
+                cst[u] = buffer_load<double>(crsrc, (uint32_t)((k * ldct + j) * 8));
+        }
+    };
+    auto store_c = [&](double *to) {
+#pragma unroll
+        for (int u = 0; u < NB; ++u) {
+            const int e = threadIdx.x + kWG * u;
+            to[e / kCols * kLd + e % kCols] = cst[u];
+        }
+    };
+    load_c(0);
+#pragma unroll
+    for (int b = 0; b < kLcSteps; ++b) load_x(ring[b]);
+    store_c(sc[0]);
+    load_c(1);
+    for (int c = 0; c < nchunks; ++c) {
+        __syncthreads();
+        // the other buffer was last read before this barrier
+        store_c(sc[(c + 1) & 1]);
+        load_c(c + 2);
+        const double *cb = sc[c & 1] + lk * kLd + li;
+#pragma unroll
+        for (int u = 0; u < kLcSteps; ++u) {
+            double ac[NB];
+#pragma unroll
+            for (int q = 0; q < NB; ++q) ac[q] = cb[u * 4 * kLd + q * 16];
+#pragma unroll
+            for (int g = 0; g < R2; ++g)
+#pragma unroll
+                for (int q = 0; q < NB; ++q) {
+                    acc[2 * g][q] = mfma(ac[q], ring[u][g][0], acc[2 * g][q]);
+                    acc[2 * g + 1][q] = mfma(ac[q], ring[u][g][1], acc[2 * g + 1][q]);
+                }
+            load_x(ring[u]);
+        }
+    }
+    // lane l holds (Y^T)[j0 + q*16 + l/16 + 4v][the row of its pair]
+#pragma unroll
+    for (int g = 0; g < R2; ++g)
 #pragma unroll
         for (int q = 0; q < NB; ++q)
 #pragma unroll
             for (int v = 0; v < 4; ++v) {
                 const int j = j0 + q * 16 + lk + 4 * v;
-                if (j < n) Y[row + (int64_t)j * ldy] = acc[a][q][v];
+                double *y = Y + rs[g] + (int64_t)(j < n ? j : 0) * ldy;
+                if (j >= n) continue;
+                if (ok0[g] && ok1[g])
+                    *reinterpret_cast<d2u *>(y) = d2u{acc[2 * g][q][v], acc[2 * g + 1][q][v]};
+                else if (ok0[g])
+                    y[0] = acc[2 * g][q][v];
+                else if (ok1[g])
+                    y[1] = acc[2 * g + 1][q][v];
             }
-    }
 }
 
 }  // namespace
@@ -468,39 +534,58 @@ void lincomb_mfma(int64_t nrows, int m, int n, const double *X, int64_t ldx, con
                   int64_t ldy, hipStream_t s)
 {
     if (nrows <= 0 || n <= 0) return;
-    const int nb = n <= 16 ? 1 : n <= 32 ? 2 : n <= 48 ? 3 : 4;
-    const int ntj = (n + 16 * nb - 1) / (16 * nb);
-    const int64_t nrt = (nrows + 255) / 256;
-    const unsigned g = (unsigned)(nrt * ntj);
-    const bool deep = nrows >= kRingDeepRows;
-#define GCGE_LC_LAUNCH(BM, NB)                                                              \
-    do {                                                                                    \
-        if (deep)                                                                           \
-            k_lincomb_mfma<BM, 5, NB><<<g, kWG, 0, s>>>(nrows, m, n, X, ldx, Ct, ldct,      \
-                                                        beta_scalar, beta, Y, ldy, ntj);    \
-        else                                                                                \
-            k_lincomb_mfma<BM, 4, NB><<<g, kWG, 0, s>>>(nrows, m, n, X, ldx, Ct, ldct,      \
-                                                        beta_scalar, beta, Y, ldy, ntj);    \
+    // as few column tiles of at most 9 x 16 columns as cover n, evenly wide
+    const int t16 = (n + 15) / 16;
+    const bool big = 3 * ldx + nrows >= (int64_t(1) << 29) || (int64_t)m * ldct >= (int64_t(1) << 28);
+    const int most = big ? 4 : beta_mode == 0 ? kLcMaxNB : kLcMaxNB - 1;
+    const int ntj = (t16 + most - 1) / most;
+    const int nb = big ? 4 : (t16 + ntj - 1) / ntj;
+    // 64 rows per wave for narrow tiles, while that leaves enough workgroups
+    const bool tall = !big && nb <= 4 && (nrows + 255) / 256 * ntj >= kLcTallWg;
+    const int64_t rows = tall ? 256 : 128;
+    const unsigned g = (unsigned)((nrows + rows - 1) / rows * ntj);
+#define GCGE_LC(BM, R2, NB)                                                                   \
+    do {                                                                                      \
+        if (NB == 4 && R2 == 1 && big)                                                        \
+            k_lincomb<BM, 1, 4, true><<<g, kWG, 0, s>>>(nrows, m, n, X, ldx, Ct, ldct,        \
+                                                        beta_scalar, beta, Y, ldy, ntj);      \
+        else                                                                                  \
+            k_lincomb<BM, R2, NB, false><<<g, kWG, 0, s>>>(nrows, m, n, X, ldx, Ct, ldct,     \
+                                                           beta_scalar, beta, Y, ldy, ntj);   \
     } while (0)
-#define GCGE_LC_NB(BM)                                                                      \
-    do {                                                                                    \
-        if (nb == 1)                                                                        \
-            GCGE_LC_LAUNCH(BM, 1);                                                          \
-        else if (nb == 2)                                                                   \
-            GCGE_LC_LAUNCH(BM, 2);                                                          \
-        else if (nb == 3)                                                                   \
-            GCGE_LC_LAUNCH(BM, 3);                                                          \
-        else                                                                                \
-            GCGE_LC_LAUNCH(BM, 4);                                                          \
+#define GCGE_LC_BM(R2, NB)         \
+    do {                           \
+        if (beta_mode == 0)        \
+            GCGE_LC(0, R2, NB);    \
+        else if (beta_mode == 1)   \
+            GCGE_LC(1, R2, NB);    \
+        else                       \
+            GCGE_LC(2, R2, NB);    \
     } while (0)
-    if (beta_mode == 0)
-        GCGE_LC_NB(0);
-    else if (beta_mode == 1)
-        GCGE_LC_NB(1);
-    else
-        GCGE_LC_NB(2);
-#undef GCGE_LC_NB
-#undef GCGE_LC_LAUNCH
+#define GCGE_LC_CASE(NB)           \
+    case NB:                       \
+        if (tall)                  \
+            GCGE_LC_BM(2, NB);     \
+        else                       \
+            GCGE_LC_BM(1, NB);     \
+        break
+#define GCGE_LC_WIDE(NB)           \
+    case NB: GCGE_LC_BM(1, NB); break
+    switch (nb) {
+        GCGE_LC_CASE(1);
+        GCGE_LC_CASE(2);
+        GCGE_LC_CASE(3);
+        GCGE_LC_CASE(4);
+        GCGE_LC_WIDE(5);
+        GCGE_LC_WIDE(6);
+        GCGE_LC_WIDE(7);
+        GCGE_LC_WIDE(8);
+        GCGE_LC_WIDE(9);
+    }
+#undef GCGE_LC_WIDE
+#undef GCGE_LC_CASE
+#undef GCGE_LC_BM
+#undef GCGE_LC
 }
 
 }  // namespace gcge

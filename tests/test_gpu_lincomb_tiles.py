@@ -1,0 +1,88 @@
+"""MultiVecLinearComb at the edges of its kernel's tiles: row pairs with one
+row past the end, 16-column tiles in one to several column tiles, chunks of 16
+source columns, every beta mode, against numpy.
+
+Each value is a chain of at most m multiply-adds (padding adds zeros) and the
+product with beta, so its error is below m + 2 units of roundoff of
+|x| |c| + |y beta|."""
+import ctypes as C
+
+import numpy as np
+import pytest
+
+from gcge_amd import abi, problems as P
+from gcge_amd.solver import DeviceMatrix, HipTable
+
+pytestmark = pytest.mark.gpu
+
+
+def ia(*v):
+    return (C.c_int * len(v))(*v)
+
+
+def check(table, mat, rows, m, n, mode, x_off=0, y_off=0):
+    rng = np.random.default_rng([rows, m, n, mode])
+    x, y = rng.standard_normal((rows, m)), rng.standard_normal((rows, n))
+    c = np.asfortranarray(rng.standard_normal((m + 2, n)))
+    beta = {0: None, 1: np.array([-0.75]), 2: rng.standard_normal(n)}[mode]
+    hx, hy = table.create_multivec(m + x_off, mat), table.create_multivec(n + y_off, mat)
+    table.upload(hx, x, x_off)
+    table.upload(hy, y, y_off)
+    table.slot("MultiVecLinearComb")(
+        hx, hy, 0, ia(x_off, y_off), ia(x_off + m, y_off + n), c.ctypes.data_as(abi.c_dbl_p), m + 2,
+        beta.ctypes.data_as(abi.c_dbl_p) if mode else None, 1 if mode == 2 else 0, table.ops)
+    got = table.download(hy, y_off, y_off + n, rows)
+    table.destroy_multivec(hx, m + x_off)
+    table.destroy_multivec(hy, n + y_off)
+    b = 0.0 if mode == 0 else beta
+    want = x @ c[:m] + y * b
+    bound = (m + 2) * np.finfo(float).eps * (np.abs(x) @ np.abs(c[:m]) + np.abs(y * b))
+    assert np.all(np.abs(got - want) <= bound), (rows, m, n, mode)
+
+
+@pytest.mark.parametrize("rows", [1, 2, 3, 63, 64, 65, 127, 128, 129, 255, 257, 1001])
+def test_row_edges(hip, rows):
+    table, mat = HipTable(), DeviceMatrix(P.diagonal_ccs(np.ones(rows)))
+    for m, n in ((1, 1), (4, 17), (5, 48), (16, 16), (17, 33), (33, 130)):
+        for mode in (0, 1, 2):
+            check(table, mat, rows, m, n, mode, x_off=1, y_off=m % 2)
+
+
+@pytest.mark.parametrize("n", [15, 16, 17, 48, 64, 65, 96, 112, 113, 128, 129, 144, 145, 160, 290])
+def test_column_tiles(hip, n):
+    rows = 777
+    table, mat = HipTable(), DeviceMatrix(P.diagonal_ccs(np.ones(rows)))
+    for m in (1, 15, 31, 32, 50):
+        for mode in (0, 1, 2):
+            check(table, mat, rows, m, n, mode)
+
+
+@pytest.mark.parametrize("n", [9, 30, 40, 60])
+def test_tall_tiles(hip, n):
+    """Enough rows for 64 per wave (512 workgroups of 256), odd."""
+    rows = 131073
+    table, mat = HipTable(), DeviceMatrix(P.diagonal_ccs(np.ones(rows)))
+    for m, mode in ((3, 0), (20, 1), (17, 2)):
+        check(table, mat, rows, m, n, mode)
+
+
+def test_offsets_past_32_bits(hip):
+    """2^27 rows: three columns reach past the 32-bit offsets of a load."""
+    rows = 1 << 27
+    table = HipTable()
+    mat = DeviceMatrix.grid(P.GRID_KINDS["diagonal"], 1, 0, rows, np.ones(rows))
+    hx, hy = table.create_multivec(2, mat), table.create_multivec(1, mat)
+    hip.gcge_hip_set_random_mode(abi.GCGE_HIP_RAND_DEVICE, 5)
+    table.slot("MultiVecSetRandomValue")(hx, 0, 2, table.ops)
+    hip.gcge_hip_set_random_mode(abi.GCGE_HIP_RAND_LIBC, 0)
+    c = np.array([1.25, -0.5])
+    table.slot("MultiVecLinearComb")(hx, hy, 0, ia(0, 0), ia(2, 1), c.ctypes.data_as(abi.c_dbl_p), 2,
+                                     None, 0, table.ops)
+    want = table.download(hx, 0, 1, rows)[:, 0] * c[0]
+    want += table.download(hx, 1, 2, rows)[:, 0] * c[1]
+    got = table.download(hy, 0, 1, rows)[:, 0]
+    table.destroy_multivec(hx, 2)
+    table.destroy_multivec(hy, 1)
+    got -= want
+    # two products and a sum of values below 1.25
+    assert max(got.max(), -got.min()) <= 3 * np.finfo(float).eps * 1.75
