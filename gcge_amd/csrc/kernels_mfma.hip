@@ -9,7 +9,7 @@
 // tests/test_gpu_slots.py).
 #include <hip/hip_runtime.h>
 #include <cstdint>
-#include <type_traits>
+#include <utility>
 
 #include "app_hip_internal.h"
 #include "kernels.h"
@@ -37,38 +37,34 @@ __device__ __forceinline__ d4 mfma(double a, double b, d4 c)
 }
 
 // ---------------------------------------------------------------------
-// Gram: G (m x n) = X^T Y.  A workgroup owns a TM x TN tile of G over one
-// chunk of rows; its four waves, WM along m and 4 / WM along n, own 64 x
-// 16 NB blocks (4 x NB MFMA tiles).  The default shape is 128 x 128 (WM 2,
-// NB 4); a Y side of at most 64 columns -- the block width of most
-// orthogonalization Grams -- takes 256 x 16 NB tiles (WM 4, NB = its
-// 16-column tiles), and both sides of at most 64 a 64 x 64 tile (WM 1, NB
-// 1), so the matrix cores do not multiply 128-wide zero padding.
-// Rows are staged 16 at a time through LDS, stored column-major (row index
-// fastest, padded to 17) so each 16-lane MFMA operand read covers the
-// banks once.  Each thread fetches 4 consecutive rows (one 32-byte load)
-// of its columns of each operand, and the next stage's loads are issued
-// into registers before the current stage's MFMAs, so HBM latency overlaps
-// the matrix-core work; the default shape holds 98 VGPRs + 128 AGPRs, two
-// waves per SIMD.  Partial tiles per chunk are summed by
-// sum_chunks in a fixed order (deterministic, no atomics).  Each
-// entry sums its rows in the same order whatever the shape; the chunking,
-// and so the rounding of the partial sums, follows the tile count.
+// Gram: G (m x n) = X^T Y, over one chunk of rows per workgroup, 16 rows a
+// stage through LDS; the partial tiles of the chunks are summed by sum_chunks
+// in a fixed order (deterministic, no atomics).
+//
+// Blocks of more than 64 columns on both sides: a workgroup owns a 128 x 128
+// tile of G, its four waves 64 x 64 quadrants (4 x 4 MFMA tiles).  Rows are
+// stored column-major (row index fastest, padded to 17) so each 16-lane MFMA
+// operand read covers the banks once.  Each thread fetches 4 consecutive rows
+// (one 32-byte load) of its columns of each operand, and the next stage's
+// loads are issued into registers before the current stage's MFMAs, so HBM
+// latency overlaps the matrix-core work; 98 VGPRs + 128 AGPRs, two waves per
+// SIMD, the matrix cores busy 80 % (460 x 120 at 2 M rows: 4.3 ms).  The
+// layout of the narrow kernel below, double buffered with one barrier, and
+// 160-wide tiles where they pad less (75 % busy) measured no faster.
 // ---------------------------------------------------------------------
 constexpr int kGK = 16;        // rows per stage
 constexpr int kGKP = kGK + 1;
 constexpr int kGRG = kGK / 4;  // 4-row groups per stage
 
-template <int WM, int NB>
-__global__ __launch_bounds__(kWG) void k_gram_mfma(
+__global__ __launch_bounds__(kWG) void k_gram_wide(
     int64_t nrows, int m, int n, const double *__restrict__ X, int64_t ldx,
     const double *__restrict__ Y, int64_t ldy, int tm, int tn, int64_t rows_per_chunk,
     int lower_only, double *__restrict__ partial)
 {
-    constexpr int WN = 4 / WM;
-    constexpr int TM = WM * 64, TN = WN * 16 * NB;
-    constexpr int XC = TM * kGRG / kWG;                  // X columns per thread
-    constexpr int YC = (TN * kGRG + kWG - 1) / kWG;      // Y columns per thread
+    constexpr int WN = 2, NB = 4;
+    constexpr int TM = 128, TN = 128;
+    constexpr int XC = TM * kGRG / kWG;  // X columns per thread
+    constexpr int YC = TN * kGRG / kWG;  // Y columns per thread
     __shared__ double sx[TM * kGKP];
     __shared__ double sy[TN * kGKP];
     const int64_t lb = xcd_swizzle(blockIdx.x, gridDim.x);
@@ -184,18 +180,167 @@ __global__ __launch_bounds__(kWG) void k_gram_mfma(
             }
 }
 
-// Tile shape of a Gram of m x n (see k_gram_mfma).
+// ---------------------------------------------------------------------
+// A side of at most 64 columns (the block width of most orthogonalization
+// Grams): a workgroup owns a 16 MA x 16 NB tile as wide as that side, with
+// MA chosen to pad the other least, and each of its four waves computes the
+// whole tile over 4 of a stage's 16 rows; the four sums are added through LDS
+// at the end, in order.
+//
+// 8 lanes load the 16 rows of a column, two rows each (whole 128-byte lines),
+// one stage ahead into registers and from there into the other of two LDS
+// buffers (one barrier per stage).  The row pairs of a column are permuted by
+// bits 1-3 of its index, so that 16 columns' operand reads cover the banks
+// once, without padding.
+//
+// Bound by HBM, and by the matrix cores for the padding of the narrow side to
+// 16 columns; small ones by their launches.  Waves side by side over 256 x 16
+// NB and 64 x 64 tiles, as before, multiplied zeros for up to three of four
+// waves: MEASURED
+// ---------------------------------------------------------------------
+typedef double d2 __attribute__((ext_vector_type(2)));
+typedef double d2u __attribute__((ext_vector_type(2), aligned(8)));
+
+template <int MA, int NB>
+__global__ __launch_bounds__(kWG, 2) void k_gram_narrow(
+    int64_t nrows, int m, int n, const double *__restrict__ X, int64_t ldx,
+    const double *__restrict__ Y, int64_t ldy, int tm, int64_t rows_per_chunk,
+    double *__restrict__ partial)
+{
+    constexpr int TM = 16 * MA, TN = 16 * NB;
+    constexpr int kLoads = (TM + TN + 31) / 32;  // of 8 columns, per wave
+    __shared__ double stage[2][kLoads * 32 * kGK];
+    const int64_t lb = xcd_swizzle(blockIdx.x, gridDim.x);
+    const int chunk = (int)(lb / tm), t = (int)(lb % tm);
+    const int i0 = t * TM;
+    double *out = partial + lb * (TM * TN);
+    const int wave = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
+    const int lane = threadIdx.x & 63;
+    const int li = lane & 15, lk = lane >> 4;
+    const int64_t rbeg = (int64_t)chunk * rows_per_chunk;
+    int64_t rend = rbeg + rows_per_chunk;
+    if (rend > nrows) rend = nrows;
+    const int nstages = rend > rbeg ? (int)((rend - rbeg + kGK - 1) / kGK) : 0;
+    // load u of the wave: columns 8 q .. 8 q + 7 of the tile's X and Y
+    // columns, q = 4 u + wave; columns past m or n read the last one (their
+    // results are not used)
+    const int pair = (lane & 7) ^ ((wave & 1) * 4 + (lane >> 4));
+    const double *src[kLoads];
+#pragma unroll
+    for (int u = 0; u < kLoads; ++u) {
+        const int cc = (4 * u + wave) * 8 + (lane >> 3);
+        const int ic = i0 + cc < m ? i0 + cc : m - 1;
+        const int jc = cc - TM < n ? cc - TM : n - 1;
+        src[u] = cc < TM ? X + (int64_t)ic * ldx : Y + (int64_t)jc * ldy;
+        src[u] += rbeg + 2 * pair;
+    }
+    d2 reg[kLoads];
+    auto load = [&](int s) {
+        if (s >= nstages) return;  // uniform
+        const int64_t row = (int64_t)s * kGK, left = rend - rbeg - row;
+        // (the rows' test around all loads: one around each would end in a
+        // wait for it)
+        if (left >= kGK) {
+#pragma unroll
+            for (int u = 0; u < kLoads; ++u)
+                reg[u] = *reinterpret_cast<const d2u *>(src[u] + row);
+        } else {
+#pragma unroll
+            for (int u = 0; u < kLoads; ++u) {
+                reg[u][0] = 2 * pair < left ? src[u][row] : 0.0;
+                reg[u][1] = 2 * pair + 1 < left ? src[u][row + 1] : 0.0;
+            }
+        }
+    };
+    auto store = [&](double *to) {
+#pragma unroll
+        for (int u = 0; u < kLoads; ++u)
+            *reinterpret_cast<d2 *>(to + (4 * u + wave) * 128 + lane * 2) = reg[u];
+    };
+    d4 acc[MA][NB];
+#pragma unroll
+    for (int a = 0; a < MA; ++a)
+#pragma unroll
+        for (int b = 0; b < NB; ++b) acc[a][b] = d4{0.0, 0.0, 0.0, 0.0};
+    // row 4 wave + lk of column li of a 16-column tile
+    const int at = li * kGK + ((2 * wave + (lk >> 1)) ^ (li >> 1)) * 2 + (lk & 1);
+    if (nstages > 0) {
+        load(0);
+        store(stage[0]);
+        load(1);
+    }
+    for (int s = 0; s < nstages; ++s) {
+        __syncthreads();
+        // the other buffer was last read before this barrier
+        if (s + 1 < nstages) store(stage[(s + 1) & 1]);
+        load(s + 2);
+        const double *from = stage[s & 1] + at;
+        double av[MA], bv[NB];
+#pragma unroll
+        for (int a = 0; a < MA; ++a) av[a] = from[a * 256];
+#pragma unroll
+        for (int b = 0; b < NB; ++b) bv[b] = from[(MA + b) * 256];
+#pragma unroll
+        for (int a = 0; a < MA; ++a)
+#pragma unroll
+            for (int b = 0; b < NB; ++b) acc[a][b] = mfma(av[a], bv[b], acc[a][b]);
+    }
+    // the waves' sums in order, a column of tiles at a time: waves 1 and 2
+    // leave theirs in the two buffers, then wave 3 in the first
+    auto put = [&](double *to, int b) {
+#pragma unroll
+        for (int a = 0; a < MA; ++a)
+#pragma unroll
+            for (int v = 0; v < 4; ++v) to[(a * 4 + v) * 64 + lane] = acc[a][b][v];
+    };
+    auto add = [&](const double *from, int b) {
+#pragma unroll
+        for (int a = 0; a < MA; ++a)
+#pragma unroll
+            for (int v = 0; v < 4; ++v) acc[a][b][v] += from[(a * 4 + v) * 64 + lane];
+    };
+#pragma unroll
+    for (int b = 0; b < NB; ++b) {
+        __syncthreads();
+        if (wave == 1) put(stage[0], b);
+        if (wave == 2) put(stage[1], b);
+        __syncthreads();
+        if (wave == 0) {
+            add(stage[0], b);
+            add(stage[1], b);
+        }
+        __syncthreads();
+        if (wave == 3) put(stage[0], b);
+        __syncthreads();
+        if (wave == 0) {
+            add(stage[0], b);
+#pragma unroll
+            for (int a = 0; a < MA; ++a)
+#pragma unroll
+                for (int v = 0; v < 4; ++v)
+                    out[(a * 16 + lk + 4 * v) * TN + b * 16 + li] = acc[a][b][v];
+        }
+    }
+}
+
+// Tile shape of a Gram of m x n: 128 x 128, or 16 ma x 16 nb with a side of
+// at most 64 columns, computed as its transpose (swap) when that is X's.
 struct GramShape {
-    int wm, nb;
-    int rows() const { return wm * 64; }
-    int cols() const { return (4 / wm) * 16 * nb; }
+    int ma, nb;
+    bool wide, swap;
+    int rows() const { return wide ? 128 : 16 * ma; }
+    int cols() const { return wide ? 128 : 16 * nb; }
 };
 
 GramShape gram_shape(int m, int n)
 {
-    if (m <= 64 && n <= 64) return GramShape{1, 1};
-    if (n <= 64) return GramShape{4, (n + 15) / 16};
-    return GramShape{2, 4};
+    if (n > 64 && m > 64) return GramShape{0, 0, true, false};
+    const bool swap = n > 64;
+    const int t = ((swap ? n : m) + 15) / 16, nb = ((swap ? m : n) + 15) / 16;
+    // accumulators of at most 21 tiles
+    const int most = nb <= 2 ? 8 : nb == 3 ? 7 : 5;
+    const int tm = (t + most - 1) / most;
+    return GramShape{(t + tm - 1) / tm, nb, false, swap};
 }
 
 struct GramPlanM {
@@ -208,6 +353,7 @@ struct GramPlanM {
 int64_t gram_tiles(int m, int n)
 {
     const GramShape sh = gram_shape(m, n);
+    if (sh.swap) std::swap(m, n);
     return (int64_t)((m + sh.rows() - 1) / sh.rows()) * ((n + sh.cols() - 1) / sh.cols());
 }
 
@@ -220,6 +366,7 @@ GramPlanM plan_with(int64_t nrows, int m, int n, int64_t min_rows, int64_t max_w
 {
     GramPlanM p;
     p.sh = gram_shape(m, n);
+    if (p.sh.swap) std::swap(m, n);
     p.tm = (m + p.sh.rows() - 1) / p.sh.rows();
     p.tn = (n + p.sh.cols() - 1) / p.sh.cols();
     const int64_t tiles = (int64_t)p.tm * p.tn;
@@ -276,9 +423,6 @@ TuneKey gram_key(int64_t nrows, int m, int n, bool lower_only)
 // 7.81, now 6.70; 200 -> 100 at 531 K rows 0.64 and 0.59, now 0.455; at 216 K
 // rows 0.255 before, now 0.200; 200 -> 40 at 1.4 M rows 0.66, now 0.57.
 // ---------------------------------------------------------------------
-typedef double d2 __attribute__((ext_vector_type(2)));
-typedef double d2u __attribute__((ext_vector_type(2), aligned(8)));
-
 constexpr int kLcK = 16;            // k per LDS chunk
 constexpr int kLcSteps = kLcK / 4;  // its steps, all of whose X loads are in flight
 constexpr int kLcMaxNB = 9;         // 144 accumulator registers (with beta 8: no room to spare)
@@ -475,24 +619,63 @@ void launch_gram(const GramPlanM &p, int64_t nrows, int m, int n, const double *
                  const double *Y, int64_t ldy, double *G, int ldg, bool rowmajor, bool lower_only,
                  double *partial, hipStream_t s)
 {
+    if (p.sh.swap) {
+        std::swap(m, n);
+        std::swap(X, Y);
+        std::swap(ldx, ldy);
+        rowmajor = !rowmajor;
+    }
     const int64_t nblk = (int64_t)p.nchunk * p.tm * p.tn;
-#define GCGE_GRAM(WM, NB)                                                                      \
-    k_gram_mfma<WM, NB><<<(unsigned)nblk, kWG, 0, s>>>(nrows, m, n, X, ldx, Y, ldy, p.tm, p.tn, \
-                                                       p.rows_per_chunk, lower_only ? 1 : 0,   \
-                                                       partial)
-    if (p.sh.wm == 1)
-        GCGE_GRAM(1, 1);
-    else if (p.sh.wm == 4 && p.sh.nb == 1)
-        GCGE_GRAM(4, 1);
-    else if (p.sh.wm == 4 && p.sh.nb == 2)
-        GCGE_GRAM(4, 2);
-    else if (p.sh.wm == 4 && p.sh.nb == 3)
-        GCGE_GRAM(4, 3);
-    else if (p.sh.wm == 4)
-        GCGE_GRAM(4, 4);
-    else
-        GCGE_GRAM(2, 4);
-#undef GCGE_GRAM
+#define GCGE_GRAM_MA(MA, NB)                                                                  \
+    case MA:                                                                                  \
+        k_gram_narrow<MA, NB><<<(unsigned)nblk, kWG, 0, s>>>(nrows, m, n, X, ldx, Y, ldy, p.tm, \
+                                                             p.rows_per_chunk, partial);      \
+        break
+    if (p.sh.wide) {
+        k_gram_wide<<<(unsigned)nblk, kWG, 0, s>>>(nrows, m, n, X, ldx, Y, ldy, p.tm, p.tn,
+                                                   p.rows_per_chunk, lower_only ? 1 : 0, partial);
+    } else if (p.sh.nb == 1) {
+        switch (p.sh.ma) {
+            GCGE_GRAM_MA(1, 1);
+            GCGE_GRAM_MA(2, 1);
+            GCGE_GRAM_MA(3, 1);
+            GCGE_GRAM_MA(4, 1);
+            GCGE_GRAM_MA(5, 1);
+            GCGE_GRAM_MA(6, 1);
+            GCGE_GRAM_MA(7, 1);
+            GCGE_GRAM_MA(8, 1);
+        }
+    } else if (p.sh.nb == 2) {
+        switch (p.sh.ma) {
+            GCGE_GRAM_MA(1, 2);
+            GCGE_GRAM_MA(2, 2);
+            GCGE_GRAM_MA(3, 2);
+            GCGE_GRAM_MA(4, 2);
+            GCGE_GRAM_MA(5, 2);
+            GCGE_GRAM_MA(6, 2);
+            GCGE_GRAM_MA(7, 2);
+            GCGE_GRAM_MA(8, 2);
+        }
+    } else if (p.sh.nb == 3) {
+        switch (p.sh.ma) {
+            GCGE_GRAM_MA(1, 3);
+            GCGE_GRAM_MA(2, 3);
+            GCGE_GRAM_MA(3, 3);
+            GCGE_GRAM_MA(4, 3);
+            GCGE_GRAM_MA(5, 3);
+            GCGE_GRAM_MA(6, 3);
+            GCGE_GRAM_MA(7, 3);
+        }
+    } else {
+        switch (p.sh.ma) {
+            GCGE_GRAM_MA(1, 4);
+            GCGE_GRAM_MA(2, 4);
+            GCGE_GRAM_MA(3, 4);
+            GCGE_GRAM_MA(4, 4);
+            GCGE_GRAM_MA(5, 4);
+        }
+    }
+#undef GCGE_GRAM_MA
     sum_chunks(m, n, p.tm, p.tn, p.sh.rows(), p.sh.cols(), p.nchunk, partial, G, ldg, rowmajor, s);
 }
 

@@ -47,3 +47,14 @@ def test_chunk_sums(hip, chunks, m, n):
 def test_thin_tiles(hip, rows, m, n):
     """Column tiles of 8 with remainders on both sides, thin on either side."""
     check(rows, m, n)
+
+
+@pytest.mark.parametrize("rows", [1, 15, 16, 17, 33, 129, 1000, 5001])
+def test_narrow_tiles(hip, rows):
+    """A side of 9 to 64 columns against one of up to several tiles, either
+    way round: every width of tile and stages of 16 rows with remainders.
+    (At these row counts an entry's sum is a chain of at most 512 rows per
+    wave and chunk, 4 waves and the chunks: below 530 roundings.)"""
+    for m, n in ((9, 9), (16, 10), (17, 16), (33, 17), (64, 33), (65, 64), (100, 40), (113, 48),
+                 (129, 20), (200, 60), (12, 70), (40, 150), (64, 65)):
+        check(rows, m, n)
