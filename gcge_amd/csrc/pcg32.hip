@@ -524,10 +524,15 @@ __global__ __launch_bounds__(1024) void k_finish_rr(int nc, int mode,
 // tile list.  That state (rho, stop flags, tile list, count) is double
 // buffered by iteration parity, so no kernel overwrites what its own
 // workgroups still read; the sums are those of the five-launch iteration.
-// Past kFuseMaxRows each workgroup's share of the partials grows with the
-// row count and the separate reductions are cheaper.
+// Past kFuseMaxRows that holds while the vectors are small -- up to
+// kFuseMaxRowTiles rows times tiles (48^3 with 10 columns: 1.27 against 1.16
+// ms a call, 42^3 with 40: 1.57 against 1.47; 48^3 with 60: 2.38 against 2.50)
+// -- and a column has few p.w partials for every workgroup to add (844 of
+// them, 60^3 and 27 points with 8 columns: 1.42 against 1.44 ms).
 // ---------------------------------------------------------------------
 constexpr int64_t kFuseMaxRows = 65536;
+constexpr int64_t kFuseMaxRowTiles = int64_t(384) << 10;
+constexpr int kFuseMaxParts = 512;
 
 __device__ __forceinline__ void update_xr_pw_body(int64_t bx, int64_t gx, int by, 
     int64_t n, const int *__restrict__ tiles, const int *__restrict__ ntact_p, int nparts_pw,
@@ -587,11 +592,48 @@ __global__ __launch_bounds__(kWG) void k_update_xr_pw(
                       rho, active, P, Wv, D, R, partial_rr);
 }
 
-// rho and stop flag of column c from k_update_xr_pw's partials, as
+// Calls f(c, sum) for columns c0 <= c < c0 + nc, a thread each, with the FP64
+// sum of the column's nparts partials in index order.  The workgroup copies
+// as many columns at a time as fit into LDS (contiguous in memory; an odd
+// stride keeps the threads on different banks), so a sum costs its additions
+// and one trip to memory; a thread walking its column in memory waited for it
+// partial after partial (a call on 62,500 2D rows with 20 columns: 1.21 -> 1.07
+// ms; twelve served requests of 2 K to 40 K rows: 399 -> 370 ms).
+constexpr int kStageFloats = 4096;
+
+template <typename F>
+__device__ __forceinline__ void column_sums(int c0, int nc, int nparts,
+                                            const float *__restrict__ partial, float *stage, F &&f)
+{
+    const int ld = nparts | 1;
+    const int group = kStageFloats / ld < kWG ? kStageFloats / ld : kWG;  // a thread each
+    for (int g = 0; g < nc; g += group) {
+        const int cnt = nc - g < group ? nc - g : group;
+        const float *p = partial + (int64_t)(c0 + g) * nparts;
+        for (int i = threadIdx.x; i < cnt * nparts; i += kWG)
+            stage[i / nparts * ld + i % nparts] = p[i];
+        __syncthreads();
+        if ((int)threadIdx.x < cnt) {
+            const float *q = stage + (int)threadIdx.x * ld;
+            double sum = 0.0;
+            int i = 0;
+            for (; i + 8 <= nparts; i += 8) {
+                float w[8];
+#pragma unroll
+                for (int u = 0; u < 8; ++u) w[u] = q[i + u];
+#pragma unroll
+                for (int u = 0; u < 8; ++u) sum += w[u];
+            }
+            for (; i < nparts; ++i) sum += q[i];
+            f(c0 + g + (int)threadIdx.x, sum);
+        }
+        __syncthreads();
+    }
+}
+
+// rho and stop flag of column c from the sum of k_update_xr_pw's partials, as
 // k_finish_rr forms them; a stopped column keeps its state.
-__device__ __forceinline__ void next_state(int c, int nparts_rr,
-                                           const float *__restrict__ partial_rr,
-                                           const float *__restrict__ rho_o,
+__device__ __forceinline__ void next_state(int c, double sum, const float *__restrict__ rho_o,
                                            const int *__restrict__ active_o,
                                            const float *__restrict__ init_res, float rate,
                                            float tol, float &rho_n, int &act_n)
@@ -599,8 +641,6 @@ __device__ __forceinline__ void next_state(int c, int nparts_rr,
     rho_n = rho_o[c];
     act_n = active_o[c];
     if (act_n) {
-        double sum = 0.0;
-        for (int i = 0; i < nparts_rr; ++i) sum += partial_rr[(int64_t)c * nparts_rr + i];
         const float res = (float)std::sqrt(sum);
         rho_n = (float)sum;
         act_n = (res > rate * init_res[c] && res > tol) ? 1 : 0;
@@ -615,6 +655,7 @@ __device__ __forceinline__ void update_p_rr_body(int64_t bx, int64_t gx, int by,
     int *__restrict__ active_n, const float *__restrict__ init_res, float rate, float tol,
     const float *__restrict__ R, float *__restrict__ P)
 {
+    __shared__ float stage[kStageFloats];
     __shared__ int tile_on[1024 / kC];
     __shared__ float s_beta[kC];
     __shared__ int s_on;
@@ -622,15 +663,14 @@ __device__ __forceinline__ void update_p_rr_body(int64_t bx, int64_t gx, int by,
     if (bx == 0 && by == 0) {
         for (int t = threadIdx.x; t < ntile; t += kWG) tile_on[t] = 0;
         __syncthreads();
-        for (int c = threadIdx.x; c < ntile * kC; c += kWG) {
+        column_sums(0, ntile * kC, nparts_rr, partial_rr, stage, [&](int c, double sum) {
             float r;
             int on;
-            next_state(c, nparts_rr, partial_rr, rho_o, active_o, init_res, rate, tol, r, on);
+            next_state(c, sum, rho_o, active_o, init_res, rate, tol, r, on);
             rho_n[c] = r;
             active_n[c] = on;
             if (on) tile_on[c / kC] = 1;  // benign race: all writers store 1
-        }
-        __syncthreads();
+        });
         if (threadIdx.x == 0) {
             int q = 0;
             for (int t = 0; t < ntile; ++t)
@@ -643,15 +683,13 @@ __device__ __forceinline__ void update_p_rr_body(int64_t bx, int64_t gx, int by,
     const int tile = tiles_o[k];
     if (threadIdx.x == 0) s_on = 0;
     __syncthreads();
-    if (threadIdx.x < kC) {
-        const int c = tile * kC + threadIdx.x;
+    column_sums(tile * kC, kC, nparts_rr, partial_rr, stage, [&](int c, double sum) {
         float r;
         int on;
-        next_state(c, nparts_rr, partial_rr, rho_o, active_o, init_res, rate, tol, r, on);
-        s_beta[threadIdx.x] = rho_o[c] == 0.f ? 0.f : r / rho_o[c];
+        next_state(c, sum, rho_o, active_o, init_res, rate, tol, r, on);
+        s_beta[c % kC] = rho_o[c] == 0.f ? 0.f : r / rho_o[c];
         if (on) atomicOr(&s_on, 1);
-    }
-    __syncthreads();
+    });
     if (!s_on) return;  // the tile has stopped: it leaves the list
     float beta[kC];
 #pragma unroll
@@ -1210,7 +1248,8 @@ void pcg32_solve(void *matA, void **mv_b, void **mv_x, int *start, int *end, OPS
     // three launches per iteration up to kFuseMaxRows rows, with the state
     // of iteration i in buffer i % 2 (the state the first finish wrote is
     // buffer 0); five past it
-    const bool fused = S.use_fused && n <= kFuseMaxRows;
+    const bool fused = S.use_fused && (n <= kFuseMaxRows || (n * ntile <= kFuseMaxRowTiles &&
+                                                             nparts_pw(1) <= kFuseMaxParts));
     int *tl_buf[2] = {S.tiles, S.tiles_b}, *nt_buf[2] = {S.ntact, S.ntact_b};
     int *act_buf[2] = {S.active, S.active_b};
     float *rho_buf[2] = {S.rho, S.rho_b};

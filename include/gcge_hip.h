@@ -358,10 +358,10 @@ void HIPGCG_MultiLinearSolverFree_BlockPCG32(OPS *ops);
  * captured HIP graph (default on; off while kernel timing is enabled).  No
  * counterpart in the reference; for callers that need plain stream launches. */
 void HIPGCG_BlockPCG32_SetGraphs(OPS *ops, int on);
-/* Up to 65,536 rows an inner iteration is three launches, the two
- * single-workgroup reductions being done by every workgroup of the kernel
- * that follows each (default on; same sums, so the same bits as the
- * five-launch iteration).  No counterpart in the reference. */
+/* Up to 65,536 rows, and beyond while the block is small, an inner iteration
+ * is three launches, the two single-workgroup reductions being done by every
+ * workgroup of the kernel that follows each (default on; same sums, so the
+ * same bits as the five-launch iteration).  No counterpart in the reference. */
 void HIPGCG_BlockPCG32_SetFused(OPS *ops, int on);
 
 /* ------------------------------------------------------------------ */
