@@ -598,7 +598,7 @@ __global__ __launch_bounds__(kWG) void k_update_xr_pw(
 // stride keeps the threads on different banks), so a sum costs its additions
 // and one trip to memory; a thread walking its column in memory waited for it
 // partial after partial (a call on 62,500 2D rows with 20 columns: 1.21 -> 1.07
-// ms; twelve served requests of 2 K to 40 K rows: 399 -> 370 ms).
+// ms).
 constexpr int kStageFloats = 4096;
 
 template <typename F>
