@@ -70,7 +70,7 @@ struct Profiler {
 
 // One context per host thread: a stream and the thread's staging buffers.
 // Every slot enqueues on the calling thread's stream and only slots that
-// return host data synchronize, so tables driven from different threads
+// return host data wait for it, so tables driven from different threads
 // run concurrently on the device.
 struct Ctx {
     int device = 0;
@@ -108,6 +108,11 @@ struct Ctx {
     double *small(int64_t ndouble);
     double *pinned(int64_t ndouble);
     void sync();
+    // Results that the stream's last kernel writes to pinned memory:
+    // expect() before its launch, arrived() instead of sync() behind it.
+    // Each of the n values is written once, and by nothing before that kernel.
+    double *expect(int64_t n);
+    void arrived(const double *h, int64_t n);
 };
 Ctx &ctx();
 // Frees the calling thread's context (a later call creates a new one).
