@@ -195,9 +195,9 @@ def rocprof_summary(d: str):
 # kernel that it picks for 2 M rows on MI355X; a trailing '*' matches a
 # prefix of the full kernel name)
 GEMM_KERNEL = "Cijk_Ailk_Bljk_DB_MT128x128x8_MI16x16x4x1*"
-KERNEL_OF_CLASS = {"lincomb": ["k_lincomb_mfma"], "gemm": [GEMM_KERNEL],
-                   "spmm64": ["k_spmm_sell", "k_stencil7"],
-                   "spmm32": ["k_spmm_pw", "k_stencil_pw"],
+KERNEL_OF_CLASS = {"lincomb": ["k_lincomb"], "gemm": [GEMM_KERNEL],
+                   "spmm64": ["k_spmm_sell", "k_stencil7", "k_grid27_spmm"],
+                   "spmm32": ["k_spmm_pw", "k_stencil_pw", "k_grid27_pw"],
                    "pcgvec": ["k_update_p", "k_update_xr"]}
 
 
@@ -275,8 +275,9 @@ def pmc_traffic(fetch: str, write: str, cfetch: str, cwrite: str, bench_json: st
         print(f"traffic_bytes_per_launch {cls} {meas:.6e}")
 
 
-# kernel class of the library profiler -> its MFMA kernel
-MFMA_CLASSES = {"gram": "k_gram_mfma", "lincomb": "k_lincomb_mfma", "gemm": GEMM_KERNEL}
+# kernel class of the library profiler -> its MFMA kernels
+MFMA_CLASSES = {"gram": ["k_gram_wide", "k_gram_narrow"], "lincomb": ["k_lincomb"],
+                "gemm": [GEMM_KERNEL]}
 
 
 def pmc_mfma(summary: str, bench_json: str):
@@ -300,7 +301,7 @@ def pmc_mfma(summary: str, bench_json: str):
             continue
         alg = kern[cls]["flops"] / kern[cls]["launches"]
         uu = u[1] if u is not None else float("nan")
-        print(f"{cls:8s} {kname:16s} {m[0]:10d} {m[1] * 512:12.4e} {alg:12.4e} "
+        print(f"{cls:8s} {'+'.join(kname):16s} {m[0]:10d} {m[1] * 512:12.4e} {alg:12.4e} "
               f"{m[1] * 512 / alg:6.3f} {uu:10.1f} {kern[cls]['TFs']:13.1f}")
     print("# every kernel with MFMA work: dispatches, MFMA flops per dispatch, "
           "MFMA busy cycles per dispatch, MfmaUtil (%)")

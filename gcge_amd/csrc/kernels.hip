@@ -446,7 +446,7 @@ __global__ __launch_bounds__(64) void k_sum_partials(int nparts,
 // coefficient in one launch: a driver that updates its columns one by one
 // launches three kernels per column and step, 56,640 launches of 3 us in a
 // double-precision solve of 16,384 rows in blocks of 4 (311 ms, bound by
-// their launches; 132 ms with these).
+// their launches; 132 ms with these, 108 with their results polled).
 // ---------------------------------------------------------------------
 // b y + x with the product rounded, as axpby forms it for alpha = 1
 __device__ __forceinline__ double scaled_sum(double b, double y, double x)

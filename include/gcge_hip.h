@@ -76,8 +76,9 @@ int gcge_host_GetOptionFromCommandLine(const char *name, char type, void *value,
  * general sparse matrix.  Without it, a constant-coefficient 7-point
  * operator on an n^3 grid (n <= 128, point x + n y + n^2 z, one diagonal
  * value and one neighbour value, as the stencil problems' A and B) is
- * recognised and multiplied matrix-free, with the same results bit for
- * bit. */
+ * recognised and multiplied matrix-free, and a 27-point operator on an n^3
+ * grid (n <= 256, any values) by grid position, with the same results bit
+ * for bit. */
 #define GCGE_HIP_MAT_GENERAL 2
 void *HIPCCS_Create(const gcge_ccs_mat *host, int flags);
 void HIPCCS_Destroy(void **mat);
@@ -221,7 +222,8 @@ int gcge_hip_device(void);
  *   device BlockPCG, 2: Gram (inner products, both kernels),
  *   3: LinearComb (matrix-core kernel), 4: BLAS-1, 5: vector updates of
  *   the device BlockPCG (p = r + beta p; x += alpha p, r -= alpha w with
- *   r.r), 6: LinearComb by the library GEMM (from 448 Ki rows). */
+ *   r.r), 6: LinearComb by the library GEMM (large
+ *   calls whose width its 128-column tiles fit). */
 void gcge_hip_profile_enable(int on);
 void gcge_hip_profile_reset(void);
 void gcge_hip_profile_read(int kind, int64_t *launches, double *total_ms, double *bytes,
