@@ -3,6 +3,7 @@
 #pragma once
 #include <hip/hip_runtime.h>
 
+#include <atomic>
 #include <cstdint>
 #include <mutex>
 #include <vector>
@@ -140,9 +141,20 @@ struct MV {
 struct Mat {
     static constexpr uint32_t kMagic = 0x484d5431u;  // "HMT1"
     uint32_t magic = kMagic;
+    // Another number for each matrix of the process.  What is kept beyond a
+    // call and belongs to a matrix is kept by it: a matrix created after
+    // another was destroyed may get the same addresses, of the handle and of
+    // the device arrays.
+    const uint64_t serial = next_serial();
     int64_t n = 0;
     int64_t bytes = 0;
     SellMat sell;
+
+    static uint64_t next_serial()
+    {
+        static std::atomic<uint64_t> last{0};
+        return ++last;
+    }
 };
 
 // Hash of a SELL matrix's slice pointers: equal hashes let A and B share

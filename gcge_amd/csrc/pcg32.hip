@@ -828,21 +828,21 @@ struct PCG32 {
     bool use_graphs = true;
     hipGraphExec_t gexec = nullptr;
     // everything the captured launches take by value: the launch grids
-    // (active count, block width), the matrices, the shift, the stopping
-    // rule and the row-block order; the count before the latest read bounds
-    // the first k_update_p of a group
+    // (active count, block width), the matrices (which fix the arrays'
+    // addresses and the kernels: general, by grid position or matrix-free),
+    // the shift, the stopping rule and the row-block order; the count before
+    // the latest read bounds the first k_update_p of a group
     struct GraphKey {
         int ntact = -1, ntact_prev = -1, nc = 0;
         int64_t n = 0;
-        const void *a = nullptr, *as = nullptr, *av = nullptr, *b = nullptr, *bv = nullptr;
+        uint64_t a = 0, b = 0;  // Mat::serial of A and, with a shift, of B
         float sigma = 0.f, rate = 0.f, tol = 0.f;
         bool xc = false, fused = false;
         bool operator==(const GraphKey &o) const
         {
             return ntact == o.ntact && ntact_prev == o.ntact_prev && nc == o.nc && n == o.n &&
-                   a == o.a && as == o.as &&
-                   av == o.av && b == o.b && bv == o.bv && sigma == o.sigma && rate == o.rate &&
-                   tol == o.tol && xc == o.xc && fused == o.fused;
+                   a == o.a && b == o.b && sigma == o.sigma && rate == o.rate && tol == o.tol &&
+                   xc == o.xc && fused == o.fused;
         }
     } gkey;
     void drop_graph()
@@ -1078,6 +1078,7 @@ void pcg32_solve(void *matA, void **mv_b, void **mv_x, int *start, int *end, OPS
         fail("BlockPCG32: rows wider than 32 entries are not supported", __FILE__, __LINE__);
     const SellMat *Bs = &A->sell;
     float sigma = 0.f;
+    uint64_t serial_b = 0;
     if (S.B != nullptr && S.sigma != 0.0) {
         Mat *Bm = mat_of(S.B, "BlockPCG32 B");
         if (Bm->sell.val32 == nullptr) fail("BlockPCG32: B has no FP32 copy", __FILE__, __LINE__);
@@ -1086,6 +1087,7 @@ void pcg32_solve(void *matA, void **mv_b, void **mv_x, int *start, int *end, OPS
             fail("BlockPCG32: a shift needs A and B with the same SELL row structure", __FILE__,
                  __LINE__);
         Bs = &Bm->sell;
+        serial_b = Bm->serial;
         sigma = (float)S.sigma;
     }
     const int64_t n = A->n;
@@ -1322,11 +1324,8 @@ void pcg32_solve(void *matA, void **mv_b, void **mv_x, int *start, int *end, OPS
         key.ntact = ntact;
         key.nc = nc;
         key.n = n;
-        key.a = A->sell.col;
-        key.as = A->sell.slice_ptr;
-        key.av = A->sell.val32;
-        key.b = Bs->col;
-        key.bv = vB;
+        key.a = A->serial;
+        key.b = serial_b;
         key.sigma = sigma;
         key.rate = (float)S.rate;
         key.tol = (float)S.tol;
