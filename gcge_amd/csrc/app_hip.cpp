@@ -881,15 +881,18 @@ int cholqr_pass_slot(OPS *ops, void **x, int sx, int n, void *matB, void **mv_ws
     return cholqr_pass(x, sx, n, matB, mv_ws, zero_tol, rel_tol);
 }
 
+void h_MultiVecInnerProd(char, void **, void **, int, int *, int *, double *, int, OPS *);
+
 // The column updates of a BlockPCG step (src/ops_lin_sol.c:140-437) on this
 // table's multivectors, all columns in one launch: p[:, col] = r[:, col] +
 // beta p[:, col]; then x[:, x0 + col] += alpha p[:, col], r[:, col] -= alpha
 // w[:, col] with rr[k] = r[:, col] . r[:, col] -- the arithmetic and the sums
-// of MultiVecAxpby column by column and MultiVecInnerProd 'D'.  False,
-// nothing done, when ops is not this table.
+// of MultiVecAxpby column by column and MultiVecLocalInnerProd 'D'.  False,
+// nothing done, unless the slots that these stand for are this library's
+// (tested in full: a caller may have replaced any one of them).
 bool cg_p_slot(OPS *ops, void **r, void **p, const int *cols, const double *beta, int n)
 {
-    if (ops == nullptr || ops->MatDotMultiVec != h_MatDotMultiVec) return false;
+    if (ops == nullptr || ops->MultiVecAxpby != h_MultiVecAxpby) return false;
     MV *R = mv_of(r, "BlockPCG r"), *P = mv_of(p, "BlockPCG p");
     if (R->nrows != P->nrows) fail("BlockPCG: row counts differ", __FILE__, __LINE__);
     CgCols c;
@@ -909,7 +912,9 @@ bool cg_p_slot(OPS *ops, void **r, void **p, const int *cols, const double *beta
 bool cg_xr_slot(OPS *ops, void **p, void **w, void **x, int x0, void **r, const int *cols,
                 const double *alpha, int n, double *rr)
 {
-    if (ops == nullptr || ops->MatDotMultiVec != h_MatDotMultiVec) return false;
+    if (ops == nullptr || ops->MultiVecAxpby != h_MultiVecAxpby ||
+        ops->MultiVecLocalInnerProd != h_MultiVecInnerProd)
+        return false;
     MV *P = mv_of(p, "BlockPCG p"), *W = mv_of(w, "BlockPCG w"), *X = mv_of(x, "BlockPCG x"),
        *R = mv_of(r, "BlockPCG r");
     if (R->nrows != P->nrows || R->nrows != W->nrows || R->nrows != X->nrows)

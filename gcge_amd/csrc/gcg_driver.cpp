@@ -36,8 +36,8 @@ int64_t pcg32_iterations(OPS *ops);
 // operators of one grid (false otherwise); app_hip.cpp.
 bool hip_stencil_residual(OPS *ops, void *A, void *B, void **x, int sx, int nc,
                           const double *lam, void **r, int sr);
-// A BlockPCG step's column updates in one launch each when ops is the HIP
-// table (false otherwise); app_hip.cpp.
+// A BlockPCG step's column updates in one launch each when the slots of ops
+// that they stand for are the HIP table's (false otherwise); app_hip.cpp.
 bool hip_cg_p(OPS *ops, void **r, void **p, const int *cols, const double *beta, int n);
 bool hip_cg_xr(OPS *ops, void **p, void **w, void **x, int x0, void **r, const int *cols,
                const double *alpha, int n, double *rr);
