@@ -7,7 +7,7 @@ import numpy as np
 import pytest
 
 import gcge_oracle as O
-from gcge_amd import abi, problems as P
+from gcge_amd import abi, problems as P, solver as S
 from gcge_amd.solver import DeviceMatrix, HipTable
 
 pytestmark = pytest.mark.gpu
@@ -110,3 +110,66 @@ def test_block_pcg_bits(hip, n, k):
         table.destroy_multivec(hx, k)
         hip.HIPGCG_MultiLinearSolverFree_BlockPCG32(table.ops)
     assert np.array_equal(out[0], out[1])
+
+
+def recognised(table, mat):
+    """Whether products with the operator run by grid position: an infinite
+    value at the first point stays infinite there, where the general kernels'
+    padding of its short row, 0 times the value, makes NaN of it."""
+    x = np.zeros((mat.n, 1))
+    x[0] = np.inf
+    return bool(np.isinf(product(table, mat, x)[0, 0]))
+
+
+# three chunks of x-lines, odd and even, and the largest side that is
+# recognised: the offsets into a column and into a tile reach furthest
+@pytest.mark.parametrize("n", [249, 250, 256])
+def test_product_bits_long_lines(hip, n):
+    table = HipTable()
+    grid, gen = operator(n, False), operator(n, True)
+    assert recognised(table, grid) and not recognised(table, gen)
+    x = np.random.default_rng(n).standard_normal((n ** 3, 2))
+    assert np.array_equal(product(table, grid, x), product(table, gen, x))
+
+
+# from 66 on a wavefront's 64 rows can lie inside an x-line, away from its ends
+@pytest.mark.parametrize("n,k", [(64, 3), (66, 9), (67, 9), (100, 9), (130, 17), (256, 1)])
+def test_block_pcg_bits_inside_lines(hip, n, k):
+    out = []
+    rng = np.random.default_rng([n, k])
+    b, x = rng.standard_normal((n ** 3, k)), rng.standard_normal((n ** 3, k))
+    for general in (False, True):
+        table = HipTable()
+        mat = operator(n, general, fp32=True)
+        assert recognised(table, mat) == (not general)
+        hb, hx = table.create_multivec(k, mat), table.create_multivec(k, mat)
+        table.upload(hb, b)
+        table.upload(hx, x)
+        hip.HIPGCG_MultiLinearSolverSetup_BlockPCG32(9, 1e-3, 1e-14, None, 0.0, table.ops)
+        abi.slot(table.ops, "MultiLinearSolver")(mat.handle, hb, hx, ia(0, 0), ia(k, k), table.ops)
+        out.append(table.download(hx, 0, k, n ** 3))
+        table.destroy_multivec(hb, k)
+        table.destroy_multivec(hx, k)
+        hip.HIPGCG_MultiLinearSolverFree_BlockPCG32(table.ops)
+    assert np.all(np.isfinite(out[0])) and np.array_equal(out[0], out[1])
+
+
+def test_uploaded_matrices_are_recognised(hip):
+    table, n = HipTable(), 9
+    A = P.varcoef27_pair(n, 1.0, np.random.default_rng(2))[0]
+    assert recognised(table, DeviceMatrix(A))
+    assert not recognised(table, DeviceMatrix(A, general=True))
+
+
+@pytest.mark.parametrize("mode,shift", [("fp64", 1), ("mixed", 0)])
+def test_solve_bits(hip, mode, shift):
+    """Whole solves by grid position and on the general 32-entry rows."""
+    A, B = P.varcoef27_pair(20, 1.0, np.random.default_rng(8))
+    bs, ni, nm = P.slepc_block_policy(20)
+    prob = P.CCSProblem("27pt_20", A, B, 20, bs, ni, nm)
+    fp32 = mode == "mixed"
+    r = [S.solve_problem(prob, mode=mode, shift=shift, rand="device", seed=1, want_vectors=True,
+                         mats=(DeviceMatrix(A, fp32, general), DeviceMatrix(B, fp32)))
+         for general in (False, True)]
+    assert r[0].nev_conv >= 20 and r[0].num_iter == r[1].num_iter
+    assert np.array_equal(r[0].eval, r[1].eval) and np.array_equal(r[0].evec, r[1].evec)

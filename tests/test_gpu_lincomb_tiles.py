@@ -86,3 +86,40 @@ def test_offsets_past_32_bits(hip):
     got -= want
     # two products and a sum of values below 1.25
     assert max(got.max(), -got.min()) <= 3 * np.finfo(float).eps * 1.75
+
+
+@pytest.mark.parametrize("mode", [0, 1, 2])
+def test_offsets_past_32_bits_with_beta(hip, mode):
+    """More than 2^27 rows, an odd number, in two 16-column tiles, against the
+    same sums column by column (MultiVecAxpby).  Values lie in [0, 1), so each
+    side is within m + 2 units of roundoff of the sum of |c| and |beta|, and
+    one wrong value in 134 M stands out of the norm of all differences."""
+    rows, m, n = (1 << 27) + 1, 5, 18
+    table = HipTable()
+    axpby = table.slot("MultiVecAxpby")
+    mat = DeviceMatrix.grid(P.GRID_KINDS["diagonal"], 1, 0, rows, np.ones(rows))
+    hx, hy, hz = (table.create_multivec(k, mat) for k in (m, n, n))
+    hip.gcge_hip_set_random_mode(abi.GCGE_HIP_RAND_DEVICE, 5)
+    table.slot("MultiVecSetRandomValue")(hx, 0, m, table.ops)
+    table.slot("MultiVecSetRandomValue")(hy, 0, n, table.ops)
+    hip.gcge_hip_set_random_mode(abi.GCGE_HIP_RAND_LIBC, 0)
+    rng = np.random.default_rng(mode)
+    c = np.asfortranarray(rng.uniform(-1, 1, (m, n)))
+    beta = {0: None, 1: np.array([-0.75]), 2: rng.uniform(-1, 1, n)}[mode]
+    b = np.broadcast_to(0.0 if beta is None else beta, n)
+    axpby(1.0, hy, 0.0, hz, ia(0, 0), ia(n, n), table.ops)
+    for j in range(n):
+        axpby(0.0, None, b[j], hz, ia(j, j), ia(j + 1, j + 1), table.ops)
+        for k in range(m):
+            axpby(c[k, j], hx, 1.0, hz, ia(k, j), ia(k + 1, j + 1), table.ops)
+    table.slot("MultiVecLinearComb")(
+        hx, hy, 0, ia(0, 0), ia(m, n), c.ctypes.data_as(abi.c_dbl_p), m,
+        beta.ctypes.data_as(abi.c_dbl_p) if mode else None, 1 if mode == 2 else 0, table.ops)
+    axpby(-1.0, hz, 1.0, hy, ia(0, 0), ia(n, n), table.ops)
+    d = np.empty(n)
+    table.slot("MultiVecInnerProd")(b"D", hy, hy, 0, ia(0, 0), ia(n, n),
+                                    d.ctypes.data_as(abi.c_dbl_p), 1, table.ops)
+    for h, k in ((hx, m), (hy, n), (hz, n)):
+        table.destroy_multivec(h, k)
+    each = 2 * (m + 2) * np.finfo(float).eps * (np.abs(c).sum(axis=0) + np.abs(b))
+    assert np.all(np.sqrt(d) <= np.sqrt(rows) * each)
