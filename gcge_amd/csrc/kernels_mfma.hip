@@ -101,7 +101,7 @@ __global__ __launch_bounds__(kWG) void k_gram_wide(
 #pragma unroll
     for (int c = 0; c < YC; ++c) {
         const int cc = cg * YC + c;
-        yok[c] = cc < TN && j0 + cc < n;
+        yok[c] = j0 + cc < n;
         yc[c] = Y + (int64_t)(yok[c] ? j0 + cc : 0) * ldy + 4 * rg;
     }
     double px[XC][4], py[YC][4];
@@ -145,12 +145,9 @@ __global__ __launch_bounds__(kWG) void k_gram_wide(
 #pragma unroll
             for (int q = 0; q < 4; ++q) sx[(cg * XC + c) * kGKP + 4 * rg + q] = px[c][q];
 #pragma unroll
-        for (int c = 0; c < YC; ++c) {
-            if (cg * YC + c < TN) {
+        for (int c = 0; c < YC; ++c)
 #pragma unroll
-                for (int q = 0; q < 4; ++q) sy[(cg * YC + c) * kGKP + 4 * rg + q] = py[c][q];
-            }
-        }
+            for (int q = 0; q < 4; ++q) sy[(cg * YC + c) * kGKP + 4 * rg + q] = py[c][q];
         __syncthreads();
         if (r0 + kGK < rend) fetch(r0 + kGK);
 #pragma unroll 2
@@ -766,7 +763,7 @@ void lincomb_mfma(int64_t nrows, int m, int n, const double *X, int64_t ldx, con
         GCGE_LC_WIDE(6);
         GCGE_LC_WIDE(7);
         GCGE_LC_WIDE(8);
-        GCGE_LC_WIDE(9);
+        case 9: GCGE_LC(0, 1, 9); break;  // without beta (kLcMaxNB)
     }
 #undef GCGE_LC_WIDE
 #undef GCGE_LC_CASE
