@@ -123,3 +123,14 @@ def test_offsets_past_32_bits_with_beta(hip, mode):
         table.destroy_multivec(h, k)
     each = 2 * (m + 2) * np.finfo(float).eps * (np.abs(c).sum(axis=0) + np.abs(b))
     assert np.all(np.sqrt(d) <= np.sqrt(rows) * each)
+
+
+# both sides of each limit of the library GEMM: 448 Ki rows, 100 source
+# columns, destination columns whose sixteens are a multiple of 8 (113-128,
+# 241-256), no beta per column
+@pytest.mark.parametrize("rows,m,n,mode", [(458752, 100, 113, 0), (458753, 101, 128, 1),
+                                           (458752, 100, 128, 2), (458751, 100, 128, 1),
+                                           (458752, 99, 128, 0), (458752, 100, 112, 1),
+                                           (458752, 100, 129, 1), (458752, 100, 241, 1)])
+def test_library_limits(hip, rows, m, n, mode):
+    check(HipTable(), DeviceMatrix(P.diagonal_ccs(np.ones(rows))), rows, m, n, mode)
