@@ -265,12 +265,15 @@ __device__ __forceinline__ void for_cut(bool cut, F &&f)
 }
 
 // w = A p over the listed 8-column tiles with the partial p.w sums, the rows
-// and sums of k_spmm_pw (pcg32.hip).  Bound by its vector instructions (216
-// multiply-adds and 144 shifts per wavefront and tile, with the masks and
-// sums about 600).  160^3, 5 tiles: 1.22 -> 0.66 ms; a whole BlockPCG call at
-// 50^3 with 33 columns 3.22 -> 2.15 ms.  One run ahead (a ring of 2) with
-// four wavefronts per SIMD, and plane-blocked workgroup orders, measured 1-2
-// % slower; loading the outer neighbours under a lane mask 1 % slower.
+// and sums of k_spmm_pw (pcg32.hip).  The coefficients are read once and stay
+// in registers over the tiles.  Bound by its vector instructions (216
+// multiply-adds and 144 shifts per wavefront and tile, 810 with the moves,
+// masks and sums, which occupy the SIMDs 66 % of the time at 160^3) and by
+// HBM (3.0 GB there, 4.5 TB/s: p is read 2.9 times).  160^3, 5 tiles: 1.22
+// -> 0.66 ms; a whole BlockPCG call at 50^3 with 33 columns 3.22 -> 2.15 ms.
+// One run ahead (a ring of 2) with four wavefronts per SIMD, and
+// plane-blocked workgroup orders, measured 1-2 % slower; loading the outer
+// neighbours under a lane mask 1 % slower.
 __global__ __launch_bounds__(kWG, 3) void k_grid27_pw(int n, int64_t nrows,
                                                       const int64_t *__restrict__ slice_ptr,
                                                       const float *__restrict__ val,

@@ -410,7 +410,7 @@ TuneKey gram_key(int64_t nrows, int m, int n, bool lower_only)
 // X is streamed from HBM into the MFMA operand registers: a lane reads two
 // consecutive rows of a column at once, the even row for one MFMA tile and
 // the odd one for another, so a step of 4 k takes R2 16-byte loads per lane;
-// they are issued 8 steps ahead (a ring of 8).  C goes through LDS, 16 k at a
+// they are issued 4 steps ahead (a ring of 4).  C goes through LDS, 16 k at a
 // time and double buffered, shared by the four waves (one barrier per 16 k;
 // rows padded so that the operand reads cover the banks once).
 //

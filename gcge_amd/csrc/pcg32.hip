@@ -513,15 +513,16 @@ __global__ __launch_bounds__(1024) void k_finish_rr(int nc, int mode,
 }
 
 // ---------------------------------------------------------------------
-// Three launches per iteration for systems of up to kFuseMaxRows rows.
-// There the fixed cost of a dependent launch outweighs the work, so the
-// two single-workgroup reductions fold into the kernels that follow them:
-// each workgroup of k_update_xr_pw forms alpha for its tile's columns from
-// the SpMM's partials (the arithmetic of k_finish_pw), and each workgroup
-// of k_update_p_rr forms rho and the stop flags of its tile's columns from
-// k_update_xr_pw's partials (the arithmetic of k_finish_rr), while its
-// workgroup (0, 0) writes the new state of every column and the compacted
-// tile list.  That state (rho, stop flags, tile list, count) is double
+// Three launches per iteration for systems of up to kFuseMaxRows rows, and
+// for larger ones with small blocks (below).  There the fixed cost of a
+// dependent launch outweighs the work, so the two single-workgroup
+// reductions fold into the kernels that follow them: each workgroup of
+// k_update_xr_pw forms alpha for its tile's columns from the SpMM's partials
+// (the arithmetic of k_finish_pw), and each workgroup of k_update_p_rr forms
+// rho and the stop flags of its tile's columns from k_update_xr_pw's
+// partials (the arithmetic of k_finish_rr), while its workgroup (0, 0)
+// writes the new state of every column and the compacted tile list.  That
+// state (rho, stop flags, tile list, count) is double
 // buffered by iteration parity, so no kernel overwrites what its own
 // workgroups still read; the sums are those of the five-launch iteration.
 // Past kFuseMaxRows that holds while the vectors are small -- up to
@@ -821,7 +822,7 @@ struct PCG32 {
     int *tiles_b = nullptr, *ntact_b = nullptr, *active_b = nullptr;
     int *h_ntact = nullptr;
     int64_t iters = 0;
-    bool use_fused = true;  // three launches per iteration up to kFuseMaxRows rows
+    bool use_fused = true;  // three launches per iteration where the rule at kFuseMaxRows allows
     // the batcher this solver's iterations join (service workers), or null
     struct PcgBatcher *batcher = nullptr;
     // kCheck inner iterations captured as one graph, for one key
@@ -1247,9 +1248,9 @@ void pcg32_solve(void *matA, void **mv_b, void **mv_x, int *start, int *end, OPS
             tune_run(pkey, 2, 0, [&](int i) { spmm_pw(i == 1, S.tiles, S.ntact, ntact); }, st);
         xc = best == 1;
     }
-    // three launches per iteration up to kFuseMaxRows rows, with the state
-    // of iteration i in buffer i % 2 (the state the first finish wrote is
-    // buffer 0); five past it
+    // three launches per iteration by the rule at kFuseMaxRows, with the
+    // state of iteration i in buffer i % 2 (the state the first finish wrote
+    // is buffer 0); otherwise five
     const bool fused = S.use_fused && (n <= kFuseMaxRows || (n * ntile <= kFuseMaxRowTiles &&
                                                              nparts_pw(1) <= kFuseMaxParts));
     int *tl_buf[2] = {S.tiles, S.tiles_b}, *nt_buf[2] = {S.ntact, S.ntact_b};
