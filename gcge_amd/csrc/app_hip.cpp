@@ -649,18 +649,35 @@ void h_MultiVecAxpby(double alpha, void **x, double beta, void **y, int *start, 
 
 // Whether X[:, nr] C + Y diag(beta) (nc destination columns) runs as the
 // library GEMM instead of the matrix-core kernel (no per-column beta: a
-// plain GEMM then).  Both reach 62-67 TFLOP/s of what they multiply; the
-// library's tiles are 128 columns wide, the kernel's a multiple of 16, so the
-// library is taken where its tiles hold no more padding -- 120 columns of 460
-// at 2 M rows: 3.70 ms against 3.97 -- and the kernel elsewhere (141 columns
-// of 300 at 1 M rows: 2.59 against 1.54 ms; 220 of 460 at 2 M rows: 7.35
-// against 6.70); below 448 Ki rows or 100 source columns the kernel ties or
-// is faster.
-bool lincomb_library(const MV *X, const MV *Y, int nr, int nc, bool per_column_beta)
+// plain GEMM then).  Below 448 Ki rows, 100 source or 100 destination columns
+// the kernel ties or is faster.  Past them both reach 62-67 TFLOP/s of what
+// they multiply, the library about 7 % more where its columns are aligned.
+// Its tiles are 128 columns wide, the kernel's a multiple of 16, evenly over
+// as few as cover nc.  So the kernel is taken where its tiles hold less
+// padding (141 columns of 300 at 1 M rows: 2.59 against 1.54 ms; 220 of 460
+// at 2 M rows: 7.35 against 6.70) and the library where they hold as much:
+//  * 113-128 and 241-256 columns (120 of 460 at 2 M rows: 3.70 against 3.97);
+//  * from 512,000 rows on also 225-240, 337-368 and so on (240 of 300 at 2 M
+//    rows: 5.02 against 5.26 ms, 240 of 100 with beta: 2.49 against 2.80; at
+//    500,000 rows the kernel is up to 26 % faster).  That takes columns that
+//    start at multiples of 16 bytes (at an odd number of rows the kernel is
+//    up to 46 % faster), without beta and from few source columns of 64
+//    (1,000,002 rows, 228 columns: the kernel 18 % faster from 100 source
+//    columns, 2 % slower from 240, 6 % from 460);
+//  * of these, with beta and fewer than 224 source columns the kernel, which
+//    reads Y before its first product, loses another 3-7 % (112 of 100 at 2 M
+//    rows: 1.23 against 1.33 ms), so there it has to save more than an eighth
+//    of the library's columns.
+bool lincomb_library(const MV *X, const MV *Y, int nr, int nc, int beta_mode)
 {
-    return Y->nrows >= (int64_t(448) << 10) && nr >= 100 && (nc + 15) / 16 % 8 == 0 &&
-           !per_column_beta && Y->nrows <= INT32_MAX && X->ldd <= INT32_MAX &&
-           Y->ldd <= INT32_MAX;
+    if (Y->nrows < (int64_t(448) << 10) || nr < 100 || nc < 100 || beta_mode == 2 ||
+        Y->nrows > INT32_MAX || X->ldd > INT32_MAX || Y->ldd > INT32_MAX)
+        return false;
+    if ((nc + 15) / 16 % 8 == 0) return true;
+    const int align = beta_mode == 0 && nr < 256 ? 8 : 2;
+    if (Y->nrows < 512000 || (X->ldd | Y->ldd) % align != 0) return false;
+    const int own = lincomb_cols(nc, beta_mode), lib = (nc + 127) / 128 * 128;
+    return own >= lib || (beta_mode == 1 && nr < 224 && 8 * own >= 7 * lib);
 }
 
 // Y (nrows x nc) = X (nrows x nr) C + Y diag(beta) with C on the device:
@@ -713,7 +730,8 @@ void h_MultiVecLinearComb(void **x, void **y, int, int *start, int *end, double 
     // The library takes coef as it is (column-major, nr rows); the kernel
     // transposed and k-major (Ct[i * nc + k] = coef[i + k * ldc]).
     // Coefficients and beta go in one upload.
-    const bool library = lincomb_library(X, Y, nr, nc, beta != nullptr && incb != 0);
+    const int beta_mode = beta == nullptr ? 0 : incb == 0 ? 1 : 2;
+    const bool library = lincomb_library(X, Y, nr, nc, beta_mode);
     const int64_t ncoef = (int64_t)nr * nc;
     Ctx::Staging &g = c.staging(ncoef + nc);
     double *h = g.h;
@@ -724,17 +742,9 @@ void h_MultiVecLinearComb(void **x, void **y, int, int *start, int *end, double 
         else
             for (int i = 0; i < nr; ++i) h[(int64_t)i * nc + k] = src[i];
     }
-    int beta_mode = 0;
-    double beta_scalar = 0.0;
-    if (beta != nullptr) {
-        if (incb == 0) {
-            beta_mode = 1;
-            beta_scalar = *beta;
-        } else {
-            beta_mode = 2;
-            for (int k = 0; k < nc; ++k) h[ncoef + k] = beta[(int64_t)k * incb];
-        }
-    }
+    const double beta_scalar = beta_mode == 1 ? *beta : 0.0;
+    if (beta_mode == 2)
+        for (int k = 0; k < nc; ++k) h[ncoef + k] = beta[(int64_t)k * incb];
     double *d = g.d;
     HIPCHECK(hipMemcpyAsync(d, h, sizeof(double) * (ncoef + (beta_mode == 2 ? nc : 0)),
                             hipMemcpyHostToDevice, c.stream));
@@ -785,7 +795,7 @@ int cholqr_pass(void **x, int sx, int n, void *matB, void **mv_ws, double zero_t
     c.prof.end(ev, c.stream);
     c.stats.gram_calls++;
     c.stats.gram_flops += (double)X->nrows * n * n;
-    const bool library = lincomb_library(X, W, n, n, false);
+    const bool library = lincomb_library(X, W, n, n, 0);
     if (!cholqr_coef(n, G, n, zero_tol, rel_tol, work, C, library, flag, c.stream))
         fail("cholqr: order not handled", __FILE__, __LINE__);
     lincomb_launch(c, xs, X->ldd, X->nrows, n, n, C, library, 0, 0.0, nullptr, W->d, W->ldd);
@@ -861,7 +871,7 @@ int orth_coef_comb_slot(OPS *ops, double *Z, int n, int sp, int np, double zero_
         return 0;
     }
     memcpy(Z + (int64_t)n * sp, g.h + (int64_t)n * sp, sizeof(double) * nT);
-    const bool library = lincomb_library(V, W, n, np, false);
+    const bool library = lincomb_library(V, W, n, np, 0);
     const double *coef = Zp;
     if (!library) {
         transpose(n, np, Zp, n, Ft, np);

@@ -165,6 +165,8 @@ int64_t gram_mfma_chunk_doubles(int m, int n);
 void gram_mfma(int64_t nrows, int m, int n, const double *X, int64_t ldx, const double *Y,
                int64_t ldy, double *G, int ldg, bool rowmajor, bool lower_only, int choice,
                int64_t max_chunks, bool tune, double *partial, hipStream_t s);
+// columns that lincomb's tiles cover for n (with 32-bit offsets)
+int lincomb_cols(int n, int beta_mode);
 void lincomb_mfma(int64_t nrows, int m, int n, const double *X, int64_t ldx, const double *Ct,
                   int ldct, int beta_mode, double beta_scalar, const double *beta, double *Y,
                   int64_t ldy, hipStream_t s);

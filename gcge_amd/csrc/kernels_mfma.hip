@@ -584,7 +584,26 @@ __global__ __launch_bounds__(kWG, 2) void k_lincomb(
             }
 }
 
+// Column tiles of 16 nb columns: as few of at most 9 x 16 (8 x 16 with beta)
+// as cover n, evenly wide.
+struct LcTiles {
+    int nb, ntj;
+};
+
+LcTiles lc_tiles(int n, int beta_mode)
+{
+    const int t16 = (n + 15) / 16, most = beta_mode == 0 ? kLcMaxNB : kLcMaxNB - 1;
+    const int ntj = (t16 + most - 1) / most;
+    return LcTiles{(t16 + ntj - 1) / ntj, ntj};
+}
+
 }  // namespace
+
+int lincomb_cols(int n, int beta_mode)
+{
+    const LcTiles t = lc_tiles(n, beta_mode);
+    return 16 * t.nb * t.ntj;
+}
 
 int gram_mfma_choice(int64_t nrows, int m, int n, bool lower_only, bool *tune)
 {
@@ -717,12 +736,9 @@ void lincomb_mfma(int64_t nrows, int m, int n, const double *X, int64_t ldx, con
                   int64_t ldy, hipStream_t s)
 {
     if (nrows <= 0 || n <= 0) return;
-    // as few column tiles of at most 9 x 16 columns as cover n, evenly wide
-    const int t16 = (n + 15) / 16;
     const bool big = 3 * ldx + nrows >= (int64_t(1) << 29) || (int64_t)m * ldct >= (int64_t(1) << 28);
-    const int most = big ? 4 : beta_mode == 0 ? kLcMaxNB : kLcMaxNB - 1;
-    const int ntj = (t16 + most - 1) / most;
-    const int nb = big ? 4 : (t16 + ntj - 1) / ntj;
+    const LcTiles t = big ? LcTiles{4, (n + 63) / 64} : lc_tiles(n, beta_mode);
+    const int nb = t.nb, ntj = t.ntj;
     // 64 rows per wave for narrow tiles, while that leaves enough workgroups
     const bool tall = !big && nb <= 4 && (nrows + 255) / 256 * ntj >= kLcTallWg;
     const int64_t rows = tall ? 256 : 128;

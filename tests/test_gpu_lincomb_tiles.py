@@ -134,3 +134,54 @@ def test_offsets_past_32_bits_with_beta(hip, mode):
                                            (458752, 100, 129, 1), (458752, 100, 241, 1)])
 def test_library_limits(hip, rows, m, n, mode):
     check(HipTable(), DeviceMatrix(P.diagonal_ccs(np.ones(rows))), rows, m, n, mode)
+
+
+def launches(hip, kind):
+    n, ms, b, f = C.c_int64(), C.c_double(), C.c_double(), C.c_double()
+    hip.gcge_hip_profile_read(kind, C.byref(n), C.byref(ms), C.byref(b), C.byref(f))
+    return n.value
+
+
+# from 512,000 rows on the library also takes widths for which the kernel's
+# tiles hold as much padding (225-240, 353-368), and with beta and few source
+# columns an eighth less (112, 300); the alignment of the columns' starts, the
+# source columns and the rows on both sides of their limits
+@pytest.mark.parametrize("rows,m,n,mode,library", [
+    (512000, 100, 240, 0, True), (511999, 100, 240, 0, False), (512004, 100, 240, 0, False),
+    (512004, 255, 240, 0, False), (512004, 256, 240, 0, True), (512004, 100, 240, 1, True), (512001, 230, 240, 1, False), (512008, 230, 225, 1, True),
+    (512000, 230, 224, 1, False), (512000, 223, 224, 1, True), (512000, 224, 112, 1, False),
+    (512000, 100, 112, 1, True), (512000, 100, 112, 0, False), (512000, 99, 112, 1, False),
+    (512000, 120, 300, 1, True), (512000, 120, 300, 0, False), (512000, 120, 355, 0, True),
+    (512000, 100, 192, 1, False), (511984, 100, 225, 1, False)])
+def test_library_widths(hip, rows, m, n, mode, library):
+    """Which of the two runs, and its values against the kernel with the same
+    beta per column (never the library).  Values lie in [0, 1): each side is
+    within m + 2 units of roundoff of the sum of |c| and |beta|."""
+    table = HipTable()
+    mat = DeviceMatrix.grid(P.GRID_KINDS["diagonal"], 1, 0, rows, np.ones(rows))
+    hx, hy, hz = (table.create_multivec(k, mat) for k in (m, n, n))
+    hip.gcge_hip_set_random_mode(abi.GCGE_HIP_RAND_DEVICE, 7)
+    table.slot("MultiVecSetRandomValue")(hx, 0, m, table.ops)
+    table.slot("MultiVecSetRandomValue")(hy, 0, n, table.ops)
+    hip.gcge_hip_set_random_mode(abi.GCGE_HIP_RAND_LIBC, 0)
+    axpby, comb = table.slot("MultiVecAxpby"), table.slot("MultiVecLinearComb")
+    axpby(1.0, hy, 0.0, hz, ia(0, 0), ia(n, n), table.ops)
+    c = np.asfortranarray(np.random.default_rng(n).uniform(-1, 1, (m, n)))
+    one, each = np.array([0.625]), np.full(n, 0.625 if mode else 0.0)
+    hip.gcge_hip_profile_enable(1)
+    hip.gcge_hip_profile_reset()
+    comb(hx, hy, 0, ia(0, 0), ia(m, n), c.ctypes.data_as(abi.c_dbl_p), m,
+         one.ctypes.data_as(abi.c_dbl_p) if mode else None, 0, table.ops)
+    gemm, own = launches(hip, 6), launches(hip, 3)
+    hip.gcge_hip_profile_enable(0)
+    assert (gemm, own) == ((1, 0) if library else (0, 1))
+    comb(hx, hz, 0, ia(0, 0), ia(m, n), c.ctypes.data_as(abi.c_dbl_p), m,
+         each.ctypes.data_as(abi.c_dbl_p), 1, table.ops)
+    axpby(-1.0, hz, 1.0, hy, ia(0, 0), ia(n, n), table.ops)
+    d = np.empty(n)
+    table.slot("MultiVecInnerProd")(b"D", hy, hy, 0, ia(0, 0), ia(n, n),
+                                    d.ctypes.data_as(abi.c_dbl_p), 1, table.ops)
+    for h, k in ((hx, m), (hy, n), (hz, n)):
+        table.destroy_multivec(h, k)
+    bound = 2 * (m + 2) * np.finfo(float).eps * (np.abs(c).sum(axis=0) + each)
+    assert np.all(np.sqrt(d) <= np.sqrt(rows) * bound)
