@@ -19,6 +19,26 @@ struct alignas(32) f8 {
     float v[kC];
 };
 
+// A level of wave_sums and those below it: the lanes O apart keep H values
+// each of the 2 H that both hold.  (A level is an instance of its own: the
+// compiler does not unroll a loop over the levels of 64 values, and an array
+// that is indexed at run time lies in scratch memory, in the caller's loop
+// too.)
+template <int H, int O, int M, typename T>
+__device__ __forceinline__ void halve_sums(T (&v)[M], int &which)
+{
+    if constexpr (H > 0) {
+        const bool up = (threadIdx.x & O) != 0;
+#pragma unroll
+        for (int i = 0; i < H; ++i) {
+            const T keep = up ? v[i + H] : v[i], give = up ? v[i] : v[i + H];
+            v[i] = keep + __shfl_xor(give, O, 64);
+        }
+        which += up ? H : 0;
+        halve_sums<H / 2, O / 2>(v, which);
+    }
+}
+
 // Sums of M values per lane over the wavefront, each over the pairs
 // of lanes 32 apart, then 16, ...: the first log2(M) levels keep
 // half of the values on each side, so 8 values take 10 exchanges instead of
@@ -28,18 +48,8 @@ struct alignas(32) f8 {
 template <int M, typename T>
 __device__ __forceinline__ T wave_sums(T (&v)[M], int &which)
 {
-    const int lane = threadIdx.x & 63;
     which = 0;
-#pragma unroll
-    for (int h = M / 2, o = 32; h > 0; h >>= 1, o >>= 1) {
-        const bool up = (lane & o) != 0;
-#pragma unroll
-        for (int i = 0; i < h; ++i) {
-            const T keep = up ? v[i + h] : v[i], give = up ? v[i] : v[i + h];
-            v[i] = keep + __shfl_xor(give, o, 64);
-        }
-        which += up ? h : 0;
-    }
+    halve_sums<M / 2, 32>(v, which);
     T s = v[0];
 #pragma unroll
     for (int o = 32 / M; o > 0; o >>= 1) s += __shfl_xor(s, o, 64);
