@@ -452,6 +452,11 @@ bool spmm_grid27(const SellMat &A, const double *X, int64_t ldx, double *Y, int6
 {
     if (A.grid27_n == 0 || ncols <= 0) return false;
     const int n = A.grid27_n;
+    // From side 33 on the workgroups are more than the CUs; up to 38 the
+    // general kernel's rows still take few columns faster (one column at 33^3:
+    // 5.6 against 6.5-7.1 us, 4 at 36^3 9.2 against 8.9-9.6; at 32^3 5.6
+    // against 5.0, at 40^3 6.9 against 6.1-7.2).
+    if (n > 32 && n < 39 && ncols <= 3) return false;
     const int chunks = n <= 128 ? 1 : (n + 123) / 124;
     const int xlen = 2 * ((n + 2 * chunks - 1) / (2 * chunks));
     const int nby = (n + kPairWaves * kPairBy - 1) / (kPairWaves * kPairBy);

@@ -173,3 +173,14 @@ def test_solve_bits(hip, mode, shift):
          for general in (False, True)]
     assert r[0].nev_conv >= 20 and r[0].num_iter == r[1].num_iter
     assert np.array_equal(r[0].eval, r[1].eval) and np.array_equal(r[0].evec, r[1].evec)
+
+
+@pytest.mark.parametrize("n,few", [(32, False), (33, True), (38, True), (39, False)])
+def test_few_columns_on_small_grids(hip, n, few):
+    """Up to three columns of these sides take the general kernel."""
+    table = HipTable()
+    grid, gen = operator(n, False), operator(n, True)
+    assert recognised(table, grid) == (not few)
+    for k in (1, 3, 4, 5):
+        x = np.random.default_rng([n, k]).standard_normal((n ** 3, k))
+        assert np.array_equal(product(table, grid, x), product(table, gen, x))
