@@ -427,7 +427,10 @@ TuneKey gram_key(int64_t nrows, int m, int n, bool lower_only)
 // 300 -> 141 columns at 1.03 M rows took the library 2.59 ms and the old
 // kernel 1.84 at best, now 1.54 (58 TF/s); 460 -> 220 at 2 M rows 7.35 and
 // 7.81, now 6.70; 200 -> 100 at 531 K rows 0.64 and 0.59, now 0.455; at 216 K
-// rows 0.255 before, now 0.200; 200 -> 40 at 1.4 M rows 0.66, now 0.57.
+// rows 0.255 before, now 0.200; 200 -> 40 at 1.4 M rows 0.66, now 0.57.  A few
+// source columns into 8 to 32 at 1 M rows and more are slower, most with beta
+// per column (1 -> 8 at 4.1 M rows 0.143 before, now 0.167): loads beyond m
+// and Y read a tile at a time cost more there than they save.
 // ---------------------------------------------------------------------
 constexpr int kLcK = 16;            // k per LDS chunk
 constexpr int kLcSteps = kLcK / 4;  // its steps, all of whose X loads are in flight
