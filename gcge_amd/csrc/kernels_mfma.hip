@@ -427,10 +427,7 @@ TuneKey gram_key(int64_t nrows, int m, int n, bool lower_only)
 // 300 -> 141 columns at 1.03 M rows took the library 2.59 ms and the old
 // kernel 1.84 at best, now 1.54 (58 TF/s); 460 -> 220 at 2 M rows 7.35 and
 // 7.81, now 6.70; 200 -> 100 at 531 K rows 0.64 and 0.59, now 0.455; at 216 K
-// rows 0.255 before, now 0.200; 200 -> 40 at 1.4 M rows 0.66, now 0.57.  A few
-// source columns into 8 to 32 at 1 M rows and more are slower, most with beta
-// per column (1 -> 8 at 4.1 M rows 0.143 before, now 0.167): loads beyond m
-// and Y read a tile at a time cost more there than they save.
+// rows 0.255 before, now 0.200; 200 -> 40 at 1.4 M rows 0.66, now 0.57.
 // ---------------------------------------------------------------------
 constexpr int kLcK = 16;            // k per LDS chunk
 constexpr int kLcSteps = kLcK / 4;  // its steps, all of whose X loads are in flight
@@ -438,9 +435,15 @@ constexpr int kLcMaxNB = 9;         // 144 accumulator registers (with beta 8: n
 // Narrow tiles take 64 rows per wave from this many workgroups on: half the
 // reads of C per row (200 -> 40 columns at 1.4 M rows: 0.61 -> 0.57 ms).
 constexpr int64_t kLcTallWg = 512;
+// Up to this many 16-column tiles at most kLcK source columns take a form of
+// their own, in which nothing is read ahead of the one chunk of C: what the
+// general form reads past m costs as much as the work there (1 -> 8 columns
+// with beta per column at 4.1 M rows 167 against 142 us, 4 -> 17 with beta at
+// 2 M rows 151 against 141).
+constexpr int kLcOneNB = 2;
 
-// BIG: offsets of X or C past the 32 bits of a buffer load
-template <int BM, int R2, int NB, bool BIG>
+// BIG: offsets of X or C past the 32 bits of a buffer load; ONE: m <= kLcK
+template <int BM, int R2, int NB, bool BIG, bool ONE>
 __global__ __launch_bounds__(kWG, 2) void k_lincomb(
     int64_t nrows, int m, int n, const double *__restrict__ X, int64_t ldx,
     const double *__restrict__ Ct, int ldct, double beta_scalar,
@@ -448,7 +451,7 @@ __global__ __launch_bounds__(kWG, 2) void k_lincomb(
 {
     constexpr int kCols = 16 * NB;
     constexpr int kLd = NB % 2 == 0 ? kCols + 16 : kCols;
-    __shared__ double sc[2][kLcK * kLd];
+    __shared__ double sc[ONE ? 1 : 2][kLcK * kLd];
     const int64_t lb = xcd_swizzle(blockIdx.x, gridDim.x);
     const int j0 = (int)(lb % ntj) * kCols;
     const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
@@ -497,7 +500,7 @@ __global__ __launch_bounds__(kWG, 2) void k_lincomb(
             asm volatile("" ::: "memory");
         }
     }
-    const int nchunks = (m + kLcK - 1) / kLcK;
+    const int nchunks = ONE ? 1 : (m + kLcK - 1) / kLcK;
     d2 ring[kLcSteps][R2];
     // the next step's columns of X: those from m on lie past the buffer's end
     // and read as zero, so no load is conditional and none is waited for early
@@ -552,13 +555,15 @@ __global__ __launch_bounds__(kWG, 2) void k_lincomb(
 #pragma unroll
     for (int b = 0; b < kLcSteps; ++b) load_x(ring[b]);
     store_c(sc[0]);
-    load_c(1);
+    if constexpr (!ONE) load_c(1);
     for (int c = 0; c < nchunks; ++c) {
         __syncthreads();
-        // the other buffer was last read before this barrier
-        store_c(sc[(c + 1) & 1]);
-        load_c(c + 2);
-        const double *cb = sc[c & 1] + lk * kLd + li;
+        if constexpr (!ONE) {
+            // the other buffer was last read before this barrier
+            store_c(sc[(c + 1) & 1]);
+            load_c(c + 2);
+        }
+        const double *cb = sc[ONE ? 0 : c & 1] + lk * kLd + li;
 #pragma unroll
         for (int u = 0; u < kLcSteps; ++u) {
             double ac[NB];
@@ -571,7 +576,7 @@ __global__ __launch_bounds__(kWG, 2) void k_lincomb(
                     acc[2 * g][q] = mfma(ac[q], ring[u][g][0], acc[2 * g][q]);
                     acc[2 * g + 1][q] = mfma(ac[q], ring[u][g][1], acc[2 * g + 1][q]);
                 }
-            load_x(ring[u]);
+            if constexpr (!ONE) load_x(ring[u]);
         }
     }
     // lane l holds (Y^T)[j0 + q*16 + l/16 + 4v][the row of its pair]
@@ -752,14 +757,17 @@ void lincomb_mfma(int64_t nrows, int m, int n, const double *X, int64_t ldx, con
     const bool tall = !big && nb <= 4 && (nrows + 255) / 256 * ntj >= kLcTallWg;
     const int64_t rows = tall ? 256 : 128;
     const unsigned g = (unsigned)((nrows + rows - 1) / rows * ntj);
+#define GCGE_LC_GO(BM, R2, NB, BIG, ONE)                                                      \
+    k_lincomb<BM, R2, NB, BIG, ONE><<<g, kWG, 0, s>>>(nrows, m, n, X, ldx, Ct, ldct,          \
+                                                      beta_scalar, beta, Y, ldy, ntj)
 #define GCGE_LC(BM, R2, NB)                                                                   \
     do {                                                                                      \
         if (NB == 4 && R2 == 1 && big)                                                        \
-            k_lincomb<BM, 1, 4, true><<<g, kWG, 0, s>>>(nrows, m, n, X, ldx, Ct, ldct,        \
-                                                        beta_scalar, beta, Y, ldy, ntj);      \
+            GCGE_LC_GO(BM, 1, 4, true, false);                                                \
+        else if (NB <= kLcOneNB && m <= kLcK)                                                 \
+            GCGE_LC_GO(BM, R2, (NB <= kLcOneNB ? NB : 1), false, true);                       \
         else                                                                                  \
-            k_lincomb<BM, R2, NB, false><<<g, kWG, 0, s>>>(nrows, m, n, X, ldx, Ct, ldct,     \
-                                                           beta_scalar, beta, Y, ldy, ntj);   \
+            GCGE_LC_GO(BM, R2, NB, false, false);                                             \
     } while (0)
 #define GCGE_LC_BM(R2, NB)         \
     do {                           \
@@ -794,6 +802,7 @@ void lincomb_mfma(int64_t nrows, int m, int n, const double *X, int64_t ldx, con
 #undef GCGE_LC_CASE
 #undef GCGE_LC_BM
 #undef GCGE_LC
+#undef GCGE_LC_GO
 }
 
 }  // namespace gcge

@@ -185,3 +185,12 @@ def test_library_widths(hip, rows, m, n, mode, library):
         table.destroy_multivec(h, k)
     bound = 2 * (m + 2) * np.finfo(float).eps * (np.abs(c).sum(axis=0) + each)
     assert np.all(np.sqrt(d) <= np.sqrt(rows) * bound)
+
+
+@pytest.mark.parametrize("rows", [130, 131073])
+@pytest.mark.parametrize("n", [16, 17, 32, 33])
+def test_one_chunk_of_coefficients(hip, rows, n):
+    """At most 16 source columns into at most 32, and one more of each."""
+    table, mat = HipTable(), DeviceMatrix(P.diagonal_ccs(np.ones(rows)))
+    for m, mode in ((15, 1), (16, 0), (16, 2), (17, 1)):
+        check(table, mat, rows, m, n, mode)
